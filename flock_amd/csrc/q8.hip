@@ -23,6 +23,8 @@
 // y (q8_coop.wgsl:28-35) and each re-reads the weights; batches of 8 or more
 // tokens take the tile kernels further down, which reuse every weight block
 // for 8 tokens.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace flk {
@@ -975,6 +977,461 @@ __global__ __launch_bounds__(kQ8Threads, FLK_Q8_MM_WAVES) void q8_mm_kernel(Q8Ar
   q8_mm_finish<RT, TT>(a, acc, q, row0, tok0);
 }
 
+// ---------------------------------------------------------------------------
+// Enough tokens to fill the GPU with 64-row tiles: the same sums on the matrix
+// cores, bit for bit.
+//
+// v_mfma_f32_16x16x4f32 forms each output as the chain fma(a3, b3, fma(a2, b2,
+// fma(a1, b1, fma(a0, b0, c)))), rounded at every step, subnormals kept
+// (checked against fmaf chains on this part: equal on 65536 outputs of normal,
+// wide-range and subnormal inputs, where a single rounding differs in a third).
+// With c = 0 that is the order's dot4: the first product rounded, the other
+// three fused (c = +0 only turns a -0 into +0, which the fold into a partial
+// that starts at +0 cannot see). So one MFMA per four columns gives 16 tokens x
+// 16 rows of dot4s, and the VALU keeps what the order puts outside of dot4: d0
+// + d1, the FMA with the block's scale, and the tree over the 64 lanes.
+//
+// What bounds it: the VALU work left over. The tile kernels above spend 10 VALU
+// operations on 8 columns of an output, i.e. at most 63 TFLOP/s (measured 60);
+// here it is 2 and 64 / 256 MFMA cycles, but f32 MFMAs and VALU operations
+// overlap only in part on this part (16 x 16 x 4 alone 152 TFLOP/s; with 4 VALU
+// operations each, operands in registers: 98), and the conversions, the tree
+// and the staging add about 1.5 more per MFMA. 2048 tokens, us, VALU tiles ->
+// here: 4096 x 1024 with norm 282 -> 238, 6144 x 1024 with norm and SwiGLU 425
+// -> 362, 1024 x 2048 147 -> 107, 1024 x 3072 214 -> 165; 1000 tokens: 158 ->
+// 122, 226 -> 186, 79 -> 59, 114 -> 92. Two workgroups of 4 waves per CU with
+// 16 x 64 outputs per wave; 16 x 32 (NT = 2): 243, 406, 117, 181; 8 waves of 16
+// x 32 sharing a tile: 266, 411, 122, 172.
+//
+// Tokens are operand A (output row 4 (l / 16) + v of lane l), weight rows
+// operand B (output column l % 16), so a lane has one scale per block.
+//
+// The tree. Leaves (the order's 64 lanes; only the first L = min(64, pow2 >=
+// blocks per row) can be other than zero) are visited in bit-reversed order, in
+// which the pairwise tree with strides L/2 .. 1 is the plain recursive halving
+// of the sequence: a subtree is a contiguous run, finished before the next
+// begins, so only one pending sum per level is held. f32 addition commutes, so
+// these are the tree's own sums.
+typedef float q8f4 __attribute__((ext_vector_type(4)));
+constexpr int kMmFixed = 3;  // tree levels written out
+
+// Position in the visiting order: leaf number i (its blocks leaf(i), leaf(i) +
+// 64, ...) and the current block. Wave-uniform.
+struct Q8Walk {
+  uint32_t i, blk;
+};
+struct Q8Tree {
+  uint32_t nb, leaves, shift;
+  // At least 2^kMmFixed leaves: more leaves than blocks only add zeros.
+  __device__ __forceinline__ explicit Q8Tree(uint32_t blocks)
+      : nb(blocks), leaves(1u << kMmFixed) {
+    while (leaves < nb && leaves < (uint32_t)kQ8Lanes) leaves <<= 1;
+    shift = __clz((int)leaves) + 1;  // 32 - log2(leaves)
+  }
+  __device__ __forceinline__ uint32_t leaf(uint32_t i) const { return __brev(i) >> shift; }
+  // The next block of the order (empty leaves have none); past the last one
+  // any block index.
+  template <bool MULTI>
+  __device__ __forceinline__ Q8Walk next(Q8Walk w) const {
+    if (MULTI) {
+      if (w.blk + kQ8Lanes < nb) return Q8Walk{w.i, w.blk + kQ8Lanes};
+      while (w.i + 1 < leaves && leaf(w.i + 1) >= nb) w.i++;
+    }
+    return Q8Walk{w.i + 1, leaf(w.i + 1)};
+  }
+};
+
+// out <- the tree sum of `leaves` (a power of two >= 2^kMmFixed, at most 2^K)
+// leaves in visiting order; leaf(part) forms the next one. The lowest levels
+// are written out; level 4 is a loop that adds its one or two children to 0
+// (exact), so that no pending sum moves between registers; the sums pending at
+// levels 5 and 6 wait in LDS (`pend`, this lane's, kMmPendStride apart), which
+// costs two accesses per row tile and 32 registers less with NT = 4.
+constexpr int kMmPendStride = kQ8Threads;
+template <int NT, int K, class LEAF>
+__device__ __forceinline__ void q8_tree_sum(q8f4 (&out)[NT], uint32_t leaves, q8f4* pend,
+                                            LEAF leaf) {
+  const int n = leaves >= (1u << K) ? 2 : 1;
+  if constexpr (K == 0) {
+    leaf(out);
+  } else if constexpr (K <= kMmFixed) {
+    q8f4 in[NT];
+    q8_tree_sum<NT, K - 1>(out, leaves, pend, leaf);
+    q8_tree_sum<NT, K - 1>(in, leaves, pend, leaf);
+#pragma unroll
+    for (int t = 0; t < NT; t++) out[t] = out[t] + in[t];
+  } else if constexpr (K <= 4) {
+#pragma unroll
+    for (int t = 0; t < NT; t++) out[t] = q8f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int i = 0; i < n; i++) {
+      q8f4 in[NT];
+      q8_tree_sum<NT, K - 1>(in, leaves, pend, leaf);
+#pragma unroll
+      for (int t = 0; t < NT; t++) out[t] = out[t] + in[t];
+    }
+  } else {
+    q8f4* mine = pend + (K - 5) * NT * kMmPendStride;
+#pragma unroll 1
+    for (int i = 0; i < n; i++) {
+      q8_tree_sum<NT, K - 1>(out, leaves, pend, leaf);
+      if (i + 1 < n) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) mine[t * kMmPendStride] = out[t];
+      } else if (i > 0) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) out[t] = mine[t * kMmPendStride] + out[t];
+      }
+    }
+  }
+}
+
+// Folds one block into part[t] (FIRST: into 0): xa(t, h) gives, for columns 4j
+// + l / 16 of the block, j = 4h .. 4h + 3, this lane's token l % 16 of token
+// tile t; byte j of wq[h] is the quant of that column in row l % 16, sc that
+// row's scale.
+template <bool FIRST, int NT, class X>
+__device__ __forceinline__ void q8_mm_fold(q8f4 (&part)[NT], const uint32_t (&wq)[2], float sc,
+                                           X xa) {
+  const q8f4 zero = {0.f, 0.f, 0.f, 0.f};
+  q8f4 x[2][NT];
+  float wf[8];
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+      if (h == 0 || NT < 4) x[h][t] = xa(t, h);
+#pragma unroll
+  for (int j = 0; j < 8; j++) wf[j] = q8_quant(wq[j >> 2], j & 3);
+  // Groups of eight matrix products, then the VALU work on their results: an
+  // f32 MFMA with VALU operations between it and the next runs well below rate
+  // (four MFMAs and 16 VALU: 83 TFLOP/s interleaved, 98 grouped, operands in
+  // registers, 4 waves per SIMD), which sched_barrier keeps the compiler from
+  // doing.
+  constexpr int PG = NT >= 4 ? 1 : 4 / NT;  // word pairs per group
+#pragma unroll
+  for (int g0 = 0; g0 < 4; g0 += PG) {
+    q8f4 d[PG][2][NT];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < PG; g++)
+#pragma unroll
+      for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+          const int j = 2 * (g0 + g) + k;
+          d[g][k][t] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(x[j >> 2][t][j & 3], wf[j], zero, 0, 0, 0);
+        }
+    if (NT >= 4 && g0 == 1) {
+#pragma unroll
+      for (int t = 0; t < NT; t++) x[1][t] = xa(t, 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < PG; g++)
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          part[t][v] = __builtin_fmaf(sc, d[g][0][t][v] + d[g][1][t][v],
+                                      FIRST && g0 + g == 0 ? 0.f : part[t][v]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  // A use here, or the compiler sinks the whole chain to the tree's add and
+  // keeps every product until then.
+#pragma unroll
+  for (int t = 0; t < NT; t++) asm volatile("" : "+v"(part[t]));
+}
+
+// One output (token, row) of every lane of the wave; lanes l, l ^ 1 hold rows
+// 2i, 2i + 1 of one token. SwiGLU of (gate, up) row pairs into act, or res +
+// sum into o.
+__device__ __forceinline__ void q8_mm_store(const Q8Args& a, float out, uint32_t tok,
+                                            uint32_t row) {
+  if (a.act != nullptr) {  // uniform
+    const float up = xor_lane<1>(out);
+    if ((row & 1) == 0 && tok < a.n_tokens && row + 1 < a.n_rows)
+      a.act[(size_t)tok * (a.n_rows / 2) + row / 2] = q8_swiglu(out, up);
+  } else if (tok < a.n_tokens && row < a.n_rows) {
+    const size_t oi = (size_t)tok * a.n_rows + row;
+    if (a.res != nullptr) out = a.res[oi] + out;
+    a.o[oi] = out;
+  }
+}
+
+// The fused input of one element.
+template <int FUSE>
+__device__ __forceinline__ float q8_mm_input(float v, float y, float scale) {
+  if (FUSE == kMmNorm) return (v * scale) * y;
+  if (FUSE == kMmSwiglu) return q8_swiglu(v, y);
+  return v;
+}
+
+// Tile `f` of the list: (row tile, token tile), and how many more of the list's
+// tiles follow in the same token tile (`run`, this one included). When the row
+// tiles split evenly over the 8 XCDs, each XCD's eighth of the list is an
+// eighth of the rows, token tile by token tile, so that its share of the
+// weights stays in its own L2 while x streams.
+__device__ __forceinline__ void q8_mfma_tile(uint32_t f, uint32_t n_rt, uint32_t n_tt,
+                                             uint32_t& rt, uint32_t& tt, uint32_t& run) {
+  const uint32_t per = n_rt % 8 == 0 ? n_rt / 8 : n_rt;  // row tiles of a part
+  const uint32_t part = f / (per * n_tt), k = f % (per * n_tt);
+  tt = k / per;
+  rt = part * per + k % per;
+  run = per - k % per;
+}
+
+// A workgroup of 4 waves owns 64 rows (16 per wave) x 16 NT tokens at a time. x and the
+// weights go through LDS in chunks of CB blocks (two buffers, one barrier per
+// chunk, the next chunk's loads in flight), both transposed within a block so
+// that a lane's four k-steps are one read:
+//   x        [block][half][column % 4][token][step]  (16 bytes per lane)
+//   quants   [block][half][column % 4][row]          (4 bytes per lane; rows
+//            padded so that the four lane groups hit distinct banks)
+// Workgroups are dealt equal runs of the tile list (q8_mfma_tile); within a run
+// the row tiles of one token tile share its rmsnorm scales and the staging
+// pipeline. MULTI: the general walk
+// (rows of more than 64 blocks, or of a number that is no power of two);
+// otherwise every leaf is one block.
+template <int NT, int FUSE, bool MULTI>
+__global__ __launch_bounds__(kQ8Threads, 2) void q8_mfma_kernel(Q8Args a, uint32_t n_tt) {
+  constexpr int TH = kQ8Threads;
+  constexpr int T = 16 * NT;            // tokens
+  constexpr int R = 64;                 // rows
+  constexpr int CB = 2;                 // blocks per chunk
+  constexpr int XI = CB * T * 8 / TH;   // float4s of x a thread stages
+  static_assert(XI * TH == CB * T * 8 && CB * R * 2 == TH && T * 8 >= TH,
+                "staging covers a chunk; one quant piece per thread; x blocks uniform per load");
+  constexpr int XB = 32 * T;            // floats of a staged block of x
+  constexpr int WL = R + 16;            // words per (half, column % 4) of a block's quants
+  constexpr int WB = 8 * WL;            // words of a staged block of quants
+  constexpr int XC = CB * XB, WC = CB * WB, SC = CB * R;
+  __shared__ __align__(16) float xs[2 * XC];
+  __shared__ uint32_t ws[2 * WC];
+  __shared__ float ss[2 * SC];
+  __shared__ q8f4 s_pend[2 * NT * kMmPendStride];
+  __shared__ float s_scale[T];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lc = lane & 15, lg = lane >> 4;
+  const Q8Tree tree(a.n_cols / 32);
+  const uint32_t n_chunks = (tree.nb + CB - 1) / CB;
+  const uint32_t n_rt = (a.n_rows + R - 1) / R;
+  // This workgroup's run: an XCD's workgroups (ids equal mod 8) take
+  // neighbouring runs.
+  const uint32_t n_wg = gridDim.x;
+  const uint32_t seq = n_wg % 8 == 0 ? blockIdx.x % 8 * (n_wg / 8) + blockIdx.x / 8 : blockIdx.x;
+  const uint64_t n_tiles = (uint64_t)n_rt * n_tt;
+  uint32_t tile = (uint32_t)(seq * n_tiles / n_wg);
+  const uint32_t tile_end = (uint32_t)((seq + 1) * n_tiles / n_wg);
+#pragma unroll 1
+  while (tile < tile_end) {
+    uint32_t rt0, tt, run;
+    q8_mfma_tile(tile, n_rt, n_tt, rt0, tt, run);
+    const uint32_t rt1 = rt0 + min(run, tile_end - tile);
+    tile += rt1 - rt0;
+    const uint32_t tok0 = tt * T;
+
+    if (FUSE == kMmNorm) {
+      __syncthreads();  // the scales of the token tile before have been read
+#pragma unroll 1
+      for (int t = wave; t < T; t += TH / kWave) {
+        const uint32_t tok = min(tok0 + t, a.n_tokens - 1);
+        const float s = q8_norm_scale(a, a.x + (size_t)tok * a.n_cols);
+        if (lane == 0) s_scale[t] = s;
+      }
+      __syncthreads();
+    }
+
+    // Staging. Thread: float4 c4 of tokens x_tok(i), block i TH / 8T (x); half tid
+    // & 1 of row w_row, block wave / 2 (quants); row lane, block wave (scales, the
+    // first CB waves). A load's address is a scalar base plus a lane offset that
+    // stays the same.
+    const uint32_t c4 = tid & 7;
+    auto x_tok = [&](int i) { return (tid + TH * i) / 8 % T; };
+    auto x_blk = [](int i) { return TH * i / (8 * T); };
+    const int w_row = tid / 2 % R, w_blk = wave / (4 / CB);
+    const int s_blk = min(wave, CB - 1);
+    const char* const xbase = reinterpret_cast<const char*>(a.x + (size_t)tok0 * a.n_cols);
+    const char* const ubase =
+        reinterpret_cast<const char*>(FUSE == kMmSwiglu ? a.up + (size_t)tok0 * a.n_cols
+                                                        : a.norm_gain);
+    uint32_t xoff[XI], woff, soff;  // bytes
+    float xscale[XI];
+#pragma unroll
+    for (int i = 0; i < XI; i++) {
+      xoff[i] = min((uint32_t)x_tok(i), a.n_tokens - 1 - tok0) * (a.n_cols * 4) + 16 * c4;
+      xscale[i] = FUSE == kMmNorm ? s_scale[x_tok(i)] : 1.f;
+    }
+    const char *wbase, *sbase;
+    auto set_rows = [&](uint32_t rt) {
+      wbase = reinterpret_cast<const char*>(a.qs + (size_t)rt * R * a.n_cols);
+      sbase = reinterpret_cast<const char*>(a.scales + (size_t)rt * R * tree.nb);
+      const uint32_t last = a.n_rows - 1 - rt * R;
+      woff = min((uint32_t)w_row, last) * a.n_cols + 16 * (tid & 1);
+      soff = min((uint32_t)lane, last) * (tree.nb * 2);
+    };
+    float4 xv[XI], yv[XI];
+    uint4 wv;
+    uint16_t sv;
+    auto stage_load = [&](const uint32_t (&blks)[CB]) {
+      auto pick = [&](int e) {
+        uint32_t b = blks[0];
+#pragma unroll
+        for (int k = 1; k < CB; k++) b = e == k ? blks[k] : b;
+        return (size_t)b;
+      };
+      wv = *reinterpret_cast<const uint4*>(wbase + 32 * pick(w_blk) + woff);
+      sv = *reinterpret_cast<const uint16_t*>(sbase + 2 * pick(s_blk) + soff);
+#pragma unroll
+      for (int i = 0; i < XI; i++) {
+        const size_t b = 128 * pick(x_blk(i));
+        xv[i] = *reinterpret_cast<const float4*>(xbase + b + xoff[i]);
+        if (FUSE == kMmSwiglu) yv[i] = *reinterpret_cast<const float4*>(ubase + b + xoff[i]);
+        if (FUSE == kMmNorm) {
+          if (i > 0 && x_blk(i) == x_blk(i - 1))
+            yv[i] = yv[i - 1];
+          else
+            yv[i] = *reinterpret_cast<const float4*>(ubase + b + 16 * c4);
+        }
+      }
+    };
+    auto stage_store = [&](int buf) {
+      // 4 x 4 byte transpose: word c holds the quants of columns 4j + c.
+      const uint32_t lo = __builtin_amdgcn_perm(wv.y, wv.x, 0x05010400u);  // x0 y0 x1 y1
+      const uint32_t hi = __builtin_amdgcn_perm(wv.y, wv.x, 0x07030602u);  // x2 y2 x3 y3
+      const uint32_t lo2 = __builtin_amdgcn_perm(wv.w, wv.z, 0x05010400u);
+      const uint32_t hi2 = __builtin_amdgcn_perm(wv.w, wv.z, 0x07030602u);
+      uint32_t* d = ws + buf * WC + w_blk * WB + (tid & 1) * (4 * WL) + w_row;
+      d[0 * WL] = __builtin_amdgcn_perm(lo2, lo, 0x05040100u);
+      d[1 * WL] = __builtin_amdgcn_perm(lo2, lo, 0x07060302u);
+      d[2 * WL] = __builtin_amdgcn_perm(hi2, hi, 0x05040100u);
+      d[3 * WL] = __builtin_amdgcn_perm(hi2, hi, 0x07060302u);
+      if (wave < CB) ss[buf * SC + wave * R + lane] = q8_scale(sv);
+#pragma unroll
+      for (int i = 0; i < XI; i++) {
+        float* x = xs + buf * XC + x_blk(i) * XB + (c4 >> 2) * (XB / 2) + x_tok(i) * 4 + (c4 & 3);
+        x[0 * 4 * T] = q8_mm_input<FUSE>(xv[i].x, yv[i].x, xscale[i]);
+        x[1 * 4 * T] = q8_mm_input<FUSE>(xv[i].y, yv[i].y, xscale[i]);
+        x[2 * 4 * T] = q8_mm_input<FUSE>(xv[i].z, yv[i].z, xscale[i]);
+        x[3 * 4 * T] = q8_mm_input<FUSE>(xv[i].w, yv[i].w, xscale[i]);
+      }
+    };
+    // Requests the chunk after the one just requested: of this row tile, or the
+    // first one of the next (after the last row tile it is loaded for nothing).
+    Q8Walk sw{0, 0};
+    uint32_t rt_ld = rt0, ch_ld = n_chunks;
+    auto request = [&]() {
+      if (ch_ld == n_chunks) {
+        ch_ld = 0;
+        set_rows(rt_ld);
+        rt_ld = min(rt_ld + 1, rt1 - 1);
+        sw = Q8Walk{0, 0};
+      }
+      ch_ld++;
+      uint32_t blks[CB];
+#pragma unroll
+      for (int e = 0; e < CB; e++) {
+        blks[e] = min(sw.blk, tree.nb - 1);
+        sw = tree.next<MULTI>(sw);
+      }
+      stage_load(blks);
+    };
+    int buf = 0;
+    // The requested chunk becomes the current one, and the next is requested.
+    auto advance = [&]() {
+      buf ^= 1;
+      stage_store(buf);
+      __syncthreads();
+      request();
+    };
+    request();
+    __syncthreads();  // every wave is done with the token tile before
+    stage_store(0);
+    __syncthreads();
+    request();
+
+    const float* xrd = xs + lg * (4 * T) + lc * 4;
+    const uint32_t* wrd = ws + lg * WL + wave * 16 + lc;
+    const float* srd = ss + wave * 16 + lc;
+    uint32_t e = 0, leaf_i = 0;  // blocks used of the current chunk; next leaf
+    auto block = [&](q8f4 (&part)[NT], auto first) {
+      if (e == (uint32_t)CB) {
+        advance();
+        e = 0;
+      }
+      const float* xb = xrd + buf * XC + e * XB;
+      const uint32_t* wb = wrd + buf * WC + e * WB;
+      const uint32_t wq[2] = {wb[0], wb[4 * WL]};
+      q8_mm_fold<decltype(first)::value, NT>(part, wq, srd[buf * SC + e * R], [&](int t, int h) {
+        return *reinterpret_cast<const q8f4*>(xb + h * (XB / 2) + 64 * t);
+      });
+      e++;
+    };
+    auto leaf = [&](q8f4 (&part)[NT]) {
+      if constexpr (MULTI) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) part[t] = q8f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (uint32_t blk = tree.leaf(leaf_i++); blk < tree.nb; blk += kQ8Lanes)
+          block(part, std::false_type{});
+      } else {
+        block(part, std::true_type{});
+      }
+    };
+#pragma unroll 1
+    for (uint32_t rt = rt0; rt < rt1; rt++) {
+      if (rt != rt0) {
+        advance();
+        e = 0;
+        leaf_i = 0;
+      }
+      q8f4 part[NT];
+      q8_tree_sum<NT, 6>(part, tree.leaves, s_pend + tid, leaf);
+      // Opaque, so that the stores' addresses are not kept in registers across
+      // the row tiles.
+      uint32_t ot = tok0;
+      asm volatile("" : "+s"(ot));
+#pragma unroll
+      for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          q8_mm_store(a, part[t][v], ot + 16 * t + 4 * lg + v, rt * R + wave * 16 + lc);
+    }
+  }
+}
+
+// Whether a batch takes q8_mfma_kernel, with 64 (NT = 4) or 32 tokens per tile:
+// the choice with the least estimated time. 2 workgroups are resident per CU,
+// so the launch takes as long as ceil(tiles / 512) tiles, plus, with a norm, the
+// scales of the token tiles a run touches (a third of a 1024-column tile each).
+struct Q8MfmaPlan {
+  uint32_t nt, wg;  // nt 0: the VALU tile kernels
+};
+static Q8MfmaPlan q8_mfma_plan(uint32_t n_rows, uint32_t n_cols, uint32_t n_tokens, bool norm) {
+  constexpr uint64_t kSlots = 512;
+  const uint64_t n_rt = (n_rows + 63) / 64;
+  // In 64-token tiles: 512 of them at a time take 55 us at 1024 columns (78
+  // TFLOP/s); the VALU kernels reach 0.75 of that rate.
+  double best = 0.95 * (double)n_rows * n_tokens / (64.0 * 64.0 * kSlots) * (78.0 / 58.0);
+  Q8MfmaPlan p{0, 0};
+  for (uint32_t nt = 2; nt <= 4; nt += 2) {
+    const uint64_t n_tt = (n_tokens + 16 * nt - 1) / (16 * nt);
+    const uint64_t tiles = n_rt * n_tt;
+    const uint64_t wg = tiles < kSlots ? tiles : kSlots;
+    const uint64_t per = (tiles + wg - 1) / wg;
+    const uint64_t part = n_rt % 8 == 0 ? n_rt / 8 : n_rt;
+    const double tokens = per % part == 0 ? (double)(per / part) : (double)(per / part) + 1.5;
+    const double t = (nt == 4 ? 1.0 : 0.53) * (per + (norm ? tokens * 300.0 / n_cols : 0.0));
+    if (t < best && tiles <= 0x7fffffffu) {
+      best = t;
+      p = Q8MfmaPlan{nt, (uint32_t)wg};
+    }
+  }
+  return p;
+}
+
 // Workgroups: one resident wave of them (every CU filled to its occupancy
 // limit, so no workgroup waits for another to finish), never more than there
 // are row groups.
@@ -1084,7 +1541,31 @@ hipError_t launch_q8_matvec(const uint8_t* qs, const uint16_t* scales, const flo
                                           kMmMinWorkgroups)
     rpw *= 2;
   const uint32_t n_rg = (n_rt + rpw - 1) / rpw;
-  if (n_tokens >= FLK_Q8_MM_MIN_TOKENS && best_val == nullptr &&
+  const Q8MfmaPlan mp = n_tokens >= 64 && best_val == nullptr
+                            ? q8_mfma_plan(n_rows, n_cols, n_tokens, a.norm_gain != nullptr)
+                            : Q8MfmaPlan{0, 0};
+  if (mp.nt != 0) {
+    gx = mp.wg;
+    const uint32_t n_mtt = (n_tokens + 16 * mp.nt - 1) / (16 * mp.nt);
+    // One block per leaf: 8, 16, 32 or 64 blocks.
+    const bool multi = nb < (1u << kMmFixed) || nb > (uint32_t)kQ8Lanes || (nb & (nb - 1)) != 0;
+    auto go = [&](auto fuse) {
+      constexpr int F = decltype(fuse)::value;
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(gx), dim3(kQ8Threads), 0, st, a, n_mtt);
+      };
+      if (mp.nt == 4)
+        multi ? launch(q8_mfma_kernel<4, F, true>) : launch(q8_mfma_kernel<4, F, false>);
+      else
+        multi ? launch(q8_mfma_kernel<2, F, true>) : launch(q8_mfma_kernel<2, F, false>);
+    };
+    if (a.norm_gain != nullptr)
+      go(std::integral_constant<int, kMmNorm>{});
+    else if (a.up != nullptr)
+      go(std::integral_constant<int, kMmSwiglu>{});
+    else
+      go(std::integral_constant<int, kMmPlain>{});
+  } else if (n_tokens >= FLK_Q8_MM_MIN_TOKENS && best_val == nullptr &&
       (uint64_t)n_rg * n_tt <= 0x7fffffffu) {
     gx = n_rg * n_tt;
     const int fuse = a.norm_gain != nullptr ? kMmNorm : (a.up != nullptr ? kMmSwiglu : kMmPlain);

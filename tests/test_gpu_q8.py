@@ -168,6 +168,44 @@ def test_tile_kernels_equal_per_token_kernel_on_random_shapes():
         assert np.array_equal(big, small), (case, rows, cols, n, fuse)
 
 
+@pytest.mark.parametrize("rows,cols,n,fuse", [
+    (4096, 1024, 1000, "norm"),      # 64 x 64 tiles, one block per leaf, ragged last tokens
+    (6144, 1024, 500, "gate_up"),    # 64 x 32 tiles
+    (4097, 256, 601, "up"),          # 8 leaves; one row in the last row tile
+    (4100, 96, 700, "plain"),        # fewer blocks than the 8 leaves written out
+    (2050, 2080, 1100, "res"),       # 65 blocks: one leaf of two
+    (1000, 3072, 2100, "norm"),      # leaves of two blocks and of one; runs cross token tiles
+])
+def test_matrix_core_tiles_match_small_batches(rng, rows, cols, n, fuse):
+    """Batches that fill the GPU with 64-row tiles (q8_mfma_kernel) equal the
+    same tokens projected 7 at a time (the per-token kernel), bit for bit."""
+    w = ops.Q8Matrix.from_packed(random_packed(rng, rows, cols), rows, cols)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    x[:, 3] *= 1e-39  # subnormal products
+    aux = rng.standard_normal((n, max(rows, cols))).astype(np.float32)
+    gain = ops.DeviceBuffer.from_array(rng.normal(1, 0.1, cols).astype(np.float32))
+    n_out = rows // 2 if fuse == "gate_up" else rows
+
+    def run(t0, t1):
+        k = t1 - t0
+        xb = ops.DeviceBuffer.from_array(np.ascontiguousarray(x[t0:t1]))
+        ob = ops.DeviceBuffer.from_array(np.full(k * n_out, np.nan, np.float32))
+        if fuse == "gate_up":
+            ops.q8_gate_up_swiglu(w, xb, ob, k, norm_gain=gain, eps=oracle.QWEN3_EPS)
+        else:
+            kw = {"norm": dict(norm_gain=gain, eps=oracle.QWEN3_EPS), "plain": {}}.get(fuse)
+            if kw is None:
+                a = np.ascontiguousarray(aux[t0:t1, :cols if fuse == "up" else rows])
+                kw = {fuse: ops.DeviceBuffer.from_array(a)}
+            ops.q8_matvec_ex(w, xb, ob, k, **kw)
+        ops.sync()
+        return ob.download(k * n_out)
+
+    big = run(0, n)
+    small = np.concatenate([run(t, min(t + 7, n)) for t in range(0, n, 7)])
+    assert np.array_equal(big, small)
+
+
 def random_packed(rng, rows, cols):
     """Q8_0 bytes with random int8 quants and f16 scales around 4e-4 (what
     quantRowQ8 gives for N(0, 0.05) weights), built without the quantizer."""
