@@ -88,7 +88,10 @@ sys.path.insert(0, ROOT)
 
 METRIC = "decode-attn HBM GB/s (% peak) @32k ctx; prefill-attn TFLOP/s (% MFMA peak) @2k"
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
-FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix
+# MI355X dense fp32 matrix. Prefill attention forms each f32 product from six
+# bf16 ones (2.5 PFLOP/s), whose own ceiling is 417 TFLOP/s: fractions of this
+# peak can pass 1.
+FP32_MFMA_PEAK_TFLOPS = 157.3
 # MI355X's published fp32 vector peak; VALU rooflines divide by it. It counts
 # packed-fp32 instructions (two flops per lane per cycle), which this library
 # never emits, so its VALU code can reach at most half of it: VALU rooflines
@@ -152,7 +155,7 @@ class Workload:
         if self.bound in ("valu", "mixed"):
             out["frac_of_unpacked_valu"] = round(achieved / FP32_UNPACKED_VALU_TFLOPS, 4)
         if self.bound == "mixed":
-            out["note"] = ("flops of fp32-MFMA attention and VALU projections together, against "
+            out["note"] = ("flops of MFMA attention and fp32 projections together, against "
                            "the fp32 vector peak")
         if self.roofline_note:
             out["note"] = self.roofline_note
@@ -376,7 +379,7 @@ class Prefill2k(Workload):
     name = "prefill2k"
     unit = "TFLOP/s"
     bound = "mfma"
-    kernel = "flk_attn_prefill: prefill_kernel<128> (paired q tiles, no merge launch)"
+    kernel = "flk_attn_prefill: prefill_kernel<128> (equal runs of key tiles + prefill_merge_kernel)"
 
     def __init__(self, torch, ops, n=2048, pos0=0, layers=1):
         self.torch, self.ops = torch, ops
@@ -449,7 +452,7 @@ class Prefill2k(Workload):
     def config(self):
         return {"workload": f"causal GQA prefill, {self.n} tokens at position {self.pos0}, "
                             f"{self.L} layer(s): fused q/k RMSNorm + RoPE + K/V write, then "
-                            "fp32-MFMA flash attention",
+                            "flash attention on three-part bf16 MFMA (f32 precision)",
                 "layers": self.L, "n_queries": self.n, "pos0": self.pos0, "n_heads": H,
                 "n_kv_heads": HKV, "head_dim": D}
 
@@ -843,7 +846,7 @@ class Q8Prefill(Workload):
 class Prompt2k(Workload):
     """Time to first token: a 2048-token prompt through flock_amd.model.Model.step
     (embedding, 28 Qwen3-0.6B layers in prefill -- Q8_0 tile projections with
-    fused norms and SwiGLU, q/k norm + RoPE + K/V write, fp32-MFMA causal
+    fused norms and SwiGLU, q/k norm + RoPE + K/V write, MFMA causal
     attention -- then the head and argmax on the last row, read back)."""
 
     data = ("synthetic: random Q8_0 weights of the Qwen3-0.6B shapes (seeded quants, f16 "

@@ -331,11 +331,17 @@ int32_t flk_attn_prefill(const float* q, const float* kcache, const float* vcach
   if ((uint64_t)n_kv_heads * head_dim * 4 * 64 > 0x7FFFFFFFull)
     return fail(FLK_ERR_UNSUPPORTED, "prefill: %u kv heads x %u dims exceed a 64-row tile's 2 GiB",
                 n_kv_heads, head_dim);
-  const PrefillPlan p = prefill_plan(n_heads, n_kv_heads, head_dim, n_queries, pos0);
+  PrefillPlan p = prefill_plan(n_heads, n_kv_heads, head_dim, n_queries, pos0);
+  // A workspace that holds the f32 kernel's partials (none for many q tiles) is
+  // enough: the call then takes that kernel.
   rc = check_ws(ws, ws_bytes, prefill_ws_bytes(p, head_dim));
+  if (rc && !p.use_small) {
+    p.use_small = true;
+    rc = check_ws(ws, ws_bytes, prefill_ws_bytes(p, head_dim));
+  }
   if (rc) return rc;
   return hip_status(launch_prefill(q, kcache, vcache, o, n_heads, n_kv_heads, head_dim, n_queries,
-                                   pos0, ws, g_stream),
+                                   pos0, p, ws, g_stream),
                     "flk_attn_prefill");
 }
 

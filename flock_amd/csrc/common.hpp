@@ -272,6 +272,8 @@ hipError_t launch_decode(const float* q, const float* kcache, const float* vcach
                          const uint64_t* seq_row_off, const uint32_t* n_keys_dev,
                          const DecodeShape& s, const DecodeFused* fused, void* ws, hipStream_t st);
 
+// The f32 kernel's plan and launch (calls of little work).
+namespace f32 {
 struct PrefillPlan {
   uint32_t rows_per_tile;   // query-head rows of one work item (all share a kv head)
   uint32_t q_per_tile;      // rows_per_tile / group
@@ -289,7 +291,29 @@ uint64_t prefill_ws_bound(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_d
                           uint32_t max_queries, uint32_t max_keys);
 hipError_t launch_prefill(const float* q, const float* kcache, const float* vcache, float* o,
                           uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
-                          uint32_t n_queries, uint32_t pos0, void* ws, hipStream_t st);
+                          uint32_t n_queries, uint32_t pos0, const PrefillPlan& p, void* ws,
+                          hipStream_t st);
+}  // namespace f32
+
+struct PrefillPlan {
+  f32::PrefillPlan small;  // the f32 kernel's plan
+  bool use_small;          // and whether the call takes it
+  uint32_t q_per_tile;     // queries of a q tile (its rows all share a kv head)
+  uint32_t n_qtiles;
+  uint64_t key_tiles;      // of all q tiles of a kv head
+  bool cut;                // runs of key tiles end within q tiles
+  uint32_t wg_per_kvh;     // workgroups, each with a run of whole or cut q tiles
+  uint64_t partial_slots;  // two per workgroup when cut
+};
+PrefillPlan prefill_plan(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
+                         uint32_t n_queries, uint32_t pos0);
+uint64_t prefill_ws_bytes(const PrefillPlan& p, uint32_t head_dim);
+uint64_t prefill_ws_bound(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
+                          uint32_t max_queries, uint32_t max_keys);
+hipError_t launch_prefill(const float* q, const float* kcache, const float* vcache, float* o,
+                          uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
+                          uint32_t n_queries, uint32_t pos0, const PrefillPlan& p, void* ws,
+                          hipStream_t st);
 
 // ------------------------------------------------------------------ argmax --
 // argmax.wgsl's contract: (va, ia) beats (vb, ib) if va > vb, or va == vb and

@@ -1,261 +1,410 @@
-// Causal GQA prefill attention as tiled flash attention on fp32 MFMA.
+// Causal GQA prefill attention as tiled flash attention on the bf16 matrix
+// cores, in f32 precision (calls of little work: prefill_f32.hip).
 //
 // The reference (attention_prefill.wgsl:75-175) runs one workgroup per
 // (query, head), streams every key of that query through scalar FMAs and two
 // barrier-heavy tree reductions per 64-key tile. Here a work item is a "q
-// tile" of 64 query-head rows that share one kv head ((64 / G) queries x the
-// G heads of the group), so every 64-key K/V tile staged in LDS serves 64
-// rows, and both products run on v_mfma_f32_16x16x4f32 (f32 in, f32 out).
+// tile" of up to 128 query-head rows that share one kv head ((128 / G) queries
+// x the G heads of the group) and a range of its 64-key tiles.
 //
-// Per 64-key tile, each of 8 waves owns 16 rows (one 16-column block) and one
-// half (32 keys) of the tile; the two halves of a row keep separate online-
-// softmax states and are combined through LDS when the q tile is done:
-//   S^T = K Q^T     A = K block [16 keys x 4 dims] from LDS, B = Q^T from
-//                   registers (loaded once); out lane l, reg i holds
-//                   S^T[key 4(l/16)+i][row l%16].
-//   softmax         every column (one query-head row) lives in lanes with the
-//                   same l%16: in-lane max/sum over 16 values, then lane xor
-//                   16 and 32 (permlane swaps). Running (m, l) per lane, no
-//                   LDS.
-//   O^T += V^T P^T  B = P^T taken directly from the S^T registers (the key
-//                   order inside a k-step is permuted identically on both
-//                   operands); A = V^T read from LDS. Output row m of channel
-//                   block c is channel CB*m + c (CB = D/16), so a lane reads
-//                   its CB values of a key as contiguous float4s and, at the
-//                   end, holds 4*CB contiguous output channels.
-// The d-summation of S uses dim (D/4)*(l/16) + s at step s (any permutation
-// of the summed index is the same dot product), so each lane reads D/4
-// contiguous floats of a K row from LDS.
+// Arithmetic. f32 MFMAs run at 1/16 of the bf16 rate, so every operand is
+// split into three bf16 parts that add up to it exactly, and a product takes
+// six v_mfma_f32_32x32x16_bf16 (products of parts are exact in f32, sums are
+// f32): 2.67 times the f32 rate. What is left out is at most 2^-26 of a
+// product, below f32's own rounding; and an accumulator is rounded 6 times per
+// 16 products instead of 16.
 //
-// Each tile's K/V rows go from HBM straight into LDS (buffer_load_dwordx4
-// ... lds) while the previous tile is computed: no registers, no LDS store
-// instructions, and one wait + barrier per tile. The loads go through a
-// buffer descriptor made per tile (scalar registers): a lane's offsets within
-// the tile are the same for every tile, so the fetch costs no per-tile
-// address arithmetic, and rows past the last key arrive as 0. Causal bound:
-// query at absolute position p sees keys 0..p (attention_prefill.wgsl:90),
-// applied per element.
+// Per 64-key tile, each of 8 waves owns 32 rows and one half (32 keys) of the
+// tile; the two halves of a row keep separate online-softmax states and are
+// combined through LDS when the item is done:
+//   S^T = K Q^T     A = K [32 keys x 16 dims] from LDS, B = Q^T from registers
+//                   (split once per item); out lane l, reg i holds
+//                   S^T[key 8(i/4) + 4(l/32) + i%4][row l%32].
+//   softmax         a query-head row lives in lanes l and l ^ 32: in-lane
+//                   max/sum over 16 values. Running (m, l) per lane, no LDS.
+//   O^T += V^T P^T  B = P^T split from the S^T registers (the key order inside
+//                   a step is permuted alike on both operands); A = V^T from
+//                   LDS. Lane l, reg i of channel block c holds channel 32c +
+//                   8(i/4) + 4(l/32) + i%4 of row l%32.
+// 32-row blocks: each 3 KB of K or V parts read from LDS serve 6 MFMAs, i.e.
+// half of the LDS read rate; 16-row blocks would need all of it.
 //
-// Scheduling (1-D grid, workgroup id = kv head + n_kv_heads * work item, so
-// with 8 kv heads the workgroups of one kv head share an XCD and its L2):
-//   paired: work item w runs q tiles n_qtiles-1-w and w whole (their causal
-//           key counts add up to about the same for every w); writes o.
-//   split:  too few q tiles to fill the GPU (chunked prefill onto a long
-//           cache): work item (q tile, split) runs a range of key tiles and
-//           writes an (m, l, acc) partial that prefill_merge_kernel combines.
-#include <type_traits>
-
+// What bounds it: the matrix cores and the power they draw. Over a 2048-token
+// and an 8192-token prompt (16 / 8 heads of 128) MFMAs are busy 0.70 of the
+// cycles, at 1.78 GHz of 2.4 (the f32 kernel: 0.75 of the cycles). Calls with
+// their prologue, us, all of prefill on the f32 kernel -> here: 8192 tokens 2100 ->
+// 1311, 2048 tokens 153.5 -> 120.8, 64 tokens at 32768 146 -> 114, 777 at 1000
+// (32 / 8 heads of 64) 108 -> 72. Error against 64 bits: 5.2e-7 -> 4.5e-7, 3.9e-7 ->
+// 3.2e-7, 7.3e-7 -> 5.7e-7, 5.7e-7 -> 4.0e-7.
+//
+// Staging. K and V tiles come through registers (requested a whole tile
+// ahead), are split there, and go to a ring of three LDS tiles in the order
+// K0 V0 K1 V1 ...: while tile u is used, u + 1 is split and stored, spread
+// over the first half of u's matrix products; one barrier in the middle of
+// each tile's use orders the ring. Between two barriers lie the second half
+// of S, the softmax and the first half of PV, so the two waves of a SIMD drift
+// apart and one's softmax runs under the other's matrix products. Rows past
+// the last key are past the end of the loads' buffer descriptor and arrive as
+// 0. Causal bound: query at absolute position p sees keys 0..p
+// (attention_prefill.wgsl:90), applied per element.
+//
+// Scheduling: one workgroup per CU (workgroup id = kv head + n_kv_heads * w, so
+// with 8 kv heads the workgroups of one kv head share an XCD and its L2). A kv
+// head's key tiles, q tile after q tile in the order heaviest, lightest, next
+// heaviest ..., are cut into equal runs, one per workgroup (the host's table
+// `start`), whatever the shape: a prompt's causal triangle, a chunk onto a long
+// cache. Pieces of q tiles that were cut go through partials, which
+// prefill_merge_kernel combines.
 #include "prefill.hpp"
 
 namespace flk {
 
-// Requests this lane's row of q tile qt in the B-operand layout of S^T = K
-// Q^T: D/4 floats from dim (D/4) * lg.
+// One row's attention over keys key0 .. key1 - 1 in plain f32 by one wave: lane
+// = key for the scores, lane = channels for the sums. Returns (m, l) and, in
+// lane l, channels l, l + 64, ... of the unnormalised sum.
 template <int D>
-__device__ __forceinline__ void fetch_q(float4 (&qraw)[D / 16], const PrefillArgs& a,
-                                        uint32_t kvh, uint32_t qt) {
-  constexpr int DS = D / 4;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int lc = lane & 15, lg = lane >> 4;
-  const uint32_t q0 = qt * a.q_per_tile;
-  const uint32_t r = (wave & 3) * 16 + lc;
-  const uint32_t qi = q0 + r / a.group;
-  const uint32_t h = kvh * a.group + r % a.group;
-  const bool row_ok = r < a.q_per_tile * a.group && qi < a.n_queries;
-  const float4* src = reinterpret_cast<const float4*>(
-      a.q + ((size_t)(row_ok ? qi : q0) * a.n_heads + (row_ok ? h : kvh * a.group)) * D + DS * lg);
+__device__ void row_f32(const PrefillArgs& a, const float* qrow, uint32_t kvh, uint32_t key0,
+                        uint32_t key1, float& m, float& l, float (&acc)[D / 64]) {
+  const uint32_t lane = threadIdx.x & 63;
+  const size_t stride = (size_t)a.n_kv_heads * D;
+  const float* kb = a.kcache + (size_t)kvh * D;
+  const float* vb = a.vcache + (size_t)kvh * D;
+  m = -1e30f;
+  l = 0.f;
 #pragma unroll
-  for (int s4 = 0; s4 < DS / 4; s4++) qraw[s4] = src[s4];
-}
-
-// The fetched row pre-multiplied by scale * log2(e), so that S^T comes out in
-// base-2 units.
-template <int D>
-__device__ __forceinline__ void scale_q(float (&qreg)[D / 4], const float4 (&qraw)[D / 16],
-                                        const PrefillArgs& a) {
+  for (int c = 0; c < D / 64; c++) acc[c] = 0.f;
+  for (uint32_t k0 = key0; k0 < key1; k0 += 64) {
+    const uint32_t key = k0 + lane;
+    float s = -INFINITY;
+    if (key < key1) {
+      s = 0.f;
+      for (int c = 0; c < D; c++)
+        s = fmaf(kb[key * stride + c], qrow[c] * a.scale_log2e, s);
+    }
+    float mx = s;
 #pragma unroll
-  for (int s4 = 0; s4 < D / 16; s4++) {
-    qreg[4 * s4 + 0] = qraw[s4].x * a.scale_log2e;
-    qreg[4 * s4 + 1] = qraw[s4].y * a.scale_log2e;
-    qreg[4 * s4 + 2] = qraw[s4].z * a.scale_log2e;
-    qreg[4 * s4 + 3] = qraw[s4].w * a.scale_log2e;
+    for (int x = 32; x >= 1; x >>= 1) mx = fmaxf(mx, shfl_xor(mx, x));
+    if (mx > m) {  // uniform
+      const float corr = __builtin_amdgcn_exp2f(m - mx);
+      l *= corr;
+#pragma unroll
+      for (int c = 0; c < D / 64; c++) acc[c] *= corr;
+      m = mx;
+    }
+    const float p = __builtin_amdgcn_exp2f(s - m);
+    float sum = p;
+#pragma unroll
+    for (int x = 32; x >= 1; x >>= 1) sum += shfl_xor(sum, x);
+    l += sum;
+    const uint32_t n = min(key1 - k0, 64u);
+    for (uint32_t j = 0; j < n; j++) {
+      const float pj = __shfl(p, j, kWave);
+#pragma unroll
+      for (int c = 0; c < D / 64; c++)
+        acc[c] = fmaf(pj, vb[(k0 + j) * stride + 64 * c + lane], acc[c]);
+    }
   }
 }
 
-// Runs key tiles [kt0, kt1) for q tile qt of kv head kvh; writes o rows
-// (normalised) when `final`, else the partial of `slot`. Tile kt0 is (or, with
-// preloaded, already was) requested into LDS buffer pair p0, and this lane's
-// q row into qraw (the caller's). With nxt_qt >= 0, the first key tile of q
-// tile nxt_qt (key tile 0) is requested into the free buffer pair, and its q
-// rows into qraw, at the start of the last key tile, so that their latency
-// overlaps that tile and the combine; the next call passes preloaded = true
-// and that pair as its p0.
+// An item again in plain f32, for the inputs that three bf16 parts do not
+// cover. Slow, and only then:
+// - no number (an infinity or NaN in q, K or V, or a magnitude that bf16 rounds
+//   to infinity): infinite - infinite shows up as a NaN in the item's output,
+//   and what f32 arithmetic makes of such inputs (a -inf score has weight 0, an
+//   infinite v gives an infinite output) is formed here;
+// - v whose later parts fall below 2^-126, which the matrix cores read as 0: an
+//   output of less than kTinyOutput in magnitude. (Above it that costs less
+//   than 2^-24 of the output; in scores it is lost against 1.)
+constexpr float kTinyOutput = 0x1p-100f;
 template <int D>
-__device__ __forceinline__ void run_qtile(const PrefillArgs& a, const TileBuffers& lb,
-                                          uint32_t kvh, uint32_t qt, uint32_t kt0, uint32_t kt1,
-                                          bool final, size_t slot, float4 (&qraw)[D / 16],
-                                          const TileOffsets<D>& toff, uint32_t p0, bool preloaded,
-                                          int nxt_qt) {
-  constexpr int LDK = D + 4;        // padded K row in LDS (floats)
-  constexpr int DS = D / 4;         // k-steps of 4 dims for S
-  constexpr int CB = D / 16;        // channel blocks of O^T
+__device__ void item_f32(const PrefillArgs a, uint32_t kvh, uint32_t qt,
+                                      uint32_t kt0, uint32_t kt1, bool final, size_t slot) {
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (uint32_t r = wave; r < a.q_per_tile * a.group; r += kPThreads / 64) {
+    const uint32_t qi = qt * a.q_per_tile + r / a.group;
+    const uint32_t h = kvh * a.group + r % a.group;
+    if (qi >= a.n_queries) break;
+    const size_t row = ((size_t)qi * a.n_heads + h) * D;
+    float m, l, acc[D / 64];
+    row_f32<D>(a, a.q + row, kvh, kt0 * kBK, min(kt1 * kBK, a.pos0 + qi + 1), m, l, acc);
+#pragma unroll
+    for (int c = 0; c < D / 64; c++) {
+      if (final)
+        a.o[row + 64 * c + lane] = acc[c] / l;
+      else
+        a.part_acc[(slot * kRows + r) * D + 64 * c + lane] = acc[c];
+    }
+    if (!final && lane == 0) a.part_ml[slot * kRows + r] = make_float2(m, l);
+  }
+}
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
+// Key tiles on their way to LDS: this thread's share of one K and one V tile.
+template <int D>
+struct Staged {
+  using T = SplitTile<D>;
+  uint32x4 k[T::KP][2];    // slot i: float4 c and D/8 + c of a key
+  float v[T::KP][8];       // channel i of 8 keys
+};
+
+template <int D>
+struct TileLoader {
+  using T = SplitTile<D>;
+  uint32_t koff, voff;  // this thread's first bytes within a tile
+  int kdst, vdst;       // its first slots within a plane
+  uint32_t row_bytes;
+
+  __device__ __forceinline__ explicit TileLoader(uint32_t rb) : row_bytes(rb) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // K: slot c of key tid / KS (and of key 32 + that, which swizzles alike).
+    const int c = tid % T::KS, key = tid / T::KS;
+    koff = key * rb + 16 * c;
+    kdst = key * T::KS + (c ^ slot_swizzle<T::KS>(key));
+    // V: wave w has slot w of every channel; lane l channels KP l ...
+    voff = (16 * (wave >> 1) + 4 * (wave & 1)) * rb + 4 * T::KP * lane;
+    vdst = T::KP * lane * 8 + (wave ^ slot_swizzle<8>(T::KP * lane));
+  }
+  __device__ __forceinline__ int k_slot(int i) const { return kdst + 32 * T::KS * i; }
+  // The odd neighbour of an even channel: the next row, the lowest slot bit
+  // flipped.
+  __device__ __forceinline__ int v_slot(int i) const { return i ? (vdst ^ 1) + 8 : vdst; }
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const PrefillArgs& a, const float* cache,
+                                                         uint32_t kvh, uint32_t kt) const {
+    const uint32_t key0 = kt * kBK;
+    const uint32_t rows = min(a.pos0 + a.n_queries - key0, (uint32_t)kBK);
+    const size_t base = (size_t)key0 * row_bytes + (size_t)kvh * D * 4;
+    return __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(reinterpret_cast<const char*>(cache) + base), 0,
+        (rows - 1) * row_bytes + D * 4, kBufferWord3);
+  }
+  // The offsets are made opaque so that their sums with the row steps are
+  // formed at each use and not kept in registers.
+  __device__ __forceinline__ void load_k(Staged<D>& s, const PrefillArgs& a, uint32_t kvh,
+                                         uint32_t kt) const {
+    const __amdgpu_buffer_rsrc_t r = rsrc(a, a.kcache, kvh, kt);
+    uint32_t off = koff;
+    asm volatile("" : "+v"(off));
+#pragma unroll
+    for (int i = 0; i < T::KP; i++) {
+      s.k[i][0] = __builtin_amdgcn_raw_buffer_load_b128(r, off + 32 * i * row_bytes, 0, 0);
+      s.k[i][1] = __builtin_amdgcn_raw_buffer_load_b128(r, off + 32 * i * row_bytes + 2 * D, 0, 0);
+    }
+  }
+  __device__ __forceinline__ void load_v(Staged<D>& s, const PrefillArgs& a, uint32_t kvh,
+                                         uint32_t kt) const {
+    const __amdgpu_buffer_rsrc_t r = rsrc(a, a.vcache, kvh, kt);
+    uint32_t off = voff;
+    asm volatile("" : "+v"(off));
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const uint32_t o = off + ((j & 3) + 8 * (j >> 2)) * row_bytes;
+      if constexpr (T::KP == 2) {
+        const uint32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, 0);
+        s.v[0][j] = __builtin_bit_cast(float, (uint32_t)w.x);
+        s.v[1][j] = __builtin_bit_cast(float, (uint32_t)w.y);
+      } else {
+        s.v[0][j] = __builtin_bit_cast(float, (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, o, 0, 0));
+      }
+    }
+  }
+};
+
+// Step n = 4i + e of staging a tile: splits values 2e, 2e + 1 of this thread's
+// slot i; the slot's last step stores it.
+template <int D, bool V>
+__device__ __forceinline__ void stage_step(int n, const Staged<D>& s, const TileLoader<D>& ld,
+                                           uint32x4* dst, uint32x4 (&w)[3]) {
+  const int i = n / 4, e = n % 4;
+  float x, y;
+  if (V) {
+    x = s.v[i][2 * e];
+    y = s.v[i][2 * e + 1];
+  } else {
+    x = __builtin_bit_cast(float, (uint32_t)s.k[i][e / 2][2 * (e % 2)]);
+    y = __builtin_bit_cast(float, (uint32_t)s.k[i][e / 2][2 * (e % 2) + 1]);
+  }
+  uint32_t p[3];
+  split_pair(x, y, p);
+#pragma unroll
+  for (int k = 0; k < 3; k++) w[k][e] = p[k];
+  if (e == 3) {
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+      dst[k * SplitTile<D>::kPlane + (V ? ld.v_slot(i) : ld.k_slot(i))] = w[k];
+  }
+}
+
+#define FLK_SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
+
+// A lane's row of a q tile: r -> (query, head).
+template <int D>
+struct QRow {
+  uint32_t qi, h;
+  bool ok;
+
+  __device__ __forceinline__ QRow(const PrefillArgs& a, uint32_t kvh, uint32_t qt) {
+    const uint32_t r = ((threadIdx.x >> 6) & 3) * 32 + (threadIdx.x & 31);
+    qi = qt * a.q_per_tile + r / a.group;
+    h = kvh * a.group + r % a.group;
+    ok = r < a.q_per_tile * a.group && qi < a.n_queries;
+    if (!ok) {  // reads the tile's first row, writes nothing
+      qi = qt * a.q_per_tile;
+      h = kvh * a.group;
+    }
+  }
+  __device__ __forceinline__ size_t offset(const PrefillArgs& a) const {
+    return ((size_t)qi * a.n_heads + h) * D;
+  }
+  // Dims of slots 2j + lg.
+  __device__ __forceinline__ void fetch(float4 (&q)[D / 8], const PrefillArgs& a) const {
+    const int lg = (threadIdx.x >> 5) & 1;
+    const float4* src = reinterpret_cast<const float4*>(a.q + offset(a));
+#pragma unroll
+    for (int j = 0; j < D / 16; j++) {
+      q[2 * j] = src[2 * j + lg];
+      q[2 * j + 1] = src[D / 8 + 2 * j + lg];
+    }
+  }
+};
+
+// What a workgroup carries from item to item: the ring (K of the current tile,
+// its V, K of the next), and the loads in flight.
+template <int D>
+struct Pipe {
+  uint32x4 *bk, *bv, *bn;
+  Staged<D> st;
+  float4 q[D / 8];
+};
+
+// Key tiles [kt0, kt1) of q tile qt of kv head kvh; writes o rows (normalised)
+// when `final`, else the partial of `slot`. The caller has put tile kt0's K into
+// p.bk (all but the barrier) and requested its V and the q rows. Under the last
+// tile the next item's first key tile (nxt_kt) goes the same way, and q tile
+// nxt_qt's rows are requested under the combine; without a next item the caller
+// names a tile of this one.
+template <int D>
+__device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, int* s_bad, uint32_t kvh,
+                                         uint32_t qt, uint32_t kt0, uint32_t kt1, bool final,
+                                         size_t slot, const TileLoader<D>& ld, uint32_t nxt_qt,
+                                         uint32_t nxt_kt) {
+  using T = SplitTile<D>;
+  constexpr int NG = D / 16;  // groups of 6 products of S, and of PV
+  constexpr int CB = D / 32;  // channel blocks of O^T
+  constexpr int SG = NG / 4;  // groups under which a tile is split and stored
+  constexpr int BG = SG;      // group after which the barrier comes
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = wave >> 2;  // which 32 keys of every tile this wave takes
-  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const int lc = lane & 15;    // column within the 16-block = row of this lane
-  const int lg = lane >> 4;    // lane group 0..3
-  // V-read swizzle (D = 128): A-operand lane lc supplies channel 8*lc + (c ^
-  // 4*sw(lc)) of block c with sw(m) = ((m >> 2) ^ (m >> 3)) & 1, so the two
-  // float4s of a key row are read in swapped order by lanes lc and lc ^ 4 and
-  // by lanes lc and lc ^ 8: any 8 consecutive lanes cover 32 distinct banks
-  // and any 16 cover 64. Output row m of the O^T accumulators then holds
-  // channel 8*m + (c ^ 4*sw(m)); for this lane's rows m = 4*lg + j that is
-  // sw_wr.
-  const int sw_rd = CB == 8 ? ((lc >> 2) ^ (lc >> 3)) & 1 : 0;
-  const int sw_wr = CB == 8 ? (lg ^ (lg >> 1)) & 1 : 0;
-  const uint32_t n_keys_total = a.pos0 + a.n_queries;
+  const int lc = lane & 31, lg = lane >> 5;
   const uint32_t q0 = qt * a.q_per_tile;
-
-  // ---- this lane's row: r -> (query, head) -----------------------------------
-  const uint32_t r = (wave & 3) * 16 + lc;
-  const uint32_t qi = q0 + r / a.group;
-  const uint32_t h = kvh * a.group + r % a.group;
-  const bool row_ok = r < a.q_per_tile * a.group && qi < a.n_queries;
-  const uint32_t qpos = a.pos0 + qi;
-
-  auto k_buf = [&](int b) { return b ? lb.k1 : lb.k0; };
-  auto v_buf = [&](int b) { return b ? lb.v1 : lb.v0; };
-  if (!preloaded) {
-    request_tile<D>(a, k_buf(p0), v_buf(p0), kvh, kt0, n_keys_total, toff, wave_u);
-    fetch_q<D>(qraw, a, kvh, qt);
-  }
-  float qreg[D / 4];
-  scale_q<D>(qreg, qraw, a);
-  wait_vm0();       // this wave's share of tile kt0 is in LDS
-  __syncthreads();  // every wave's; the previous q tile's combine is done
-  // The next q tile's rows: in flight during the first key tile, then held.
-  if (nxt_qt >= 0) fetch_q<D>(qraw, a, kvh, (uint32_t)nxt_qt);
-  floatx4 oacc[CB];
+  const uint32_t r = (wave & 3) * 32 + lc;
+  const QRow<D> row(a, kvh, qt);
+  const uint32_t qpos = a.pos0 + row.qi;
+  const bool row_ok = row.ok;
+  uint32x4 *bk = p.bk, *bv = p.bv, *bn = p.bn;
+  Staged<D>& st = p.st;
+  uint32x4 w[3];
+  // The row's q, pre-multiplied by scale * log2(e) so that S^T comes out in
+  // base-2 units, split.
+  uint32x4 qf[NG][3];
 #pragma unroll
-  for (int c = 0; c < CB; c++) oacc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < NG; j++) {
+    const float4 x = p.q[2 * j], y = p.q[2 * j + 1];
+    const float e[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      uint32_t u[3];
+      split_pair(e[2 * i] * a.scale_log2e, e[2 * i + 1] * a.scale_log2e, u);
+#pragma unroll
+      for (int k = 0; k < 3; k++) qf[j][k][i] = u[k];
+    }
+  }
+  lds_barrier();
+
+  floatx16 oacc[CB];
+#pragma unroll
+  for (int c = 0; c < CB; c++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) oacc[c][i] = 0.f;
   // Running reference m_run (log2 units; finite, so that a masked key's
   // weight exp2(-inf - m_run) is exactly 0) and this lane's share of the
-  // denominator (its keys only; summed over the row's lanes at the end).
+  // denominator (its keys only).
   float m_run = -1e30f, l_run = 0.f;
 
   // A tile needs no causal mask when its last key is at or before the q
   // tile's first query position and every row of the q tile is live.
   const bool all_rows = a.q_per_tile * a.group == kRows && q0 + a.q_per_tile <= a.n_queries;
-  auto full_tile = [&](uint32_t key0) { return all_rows && key0 + kBK - 1 <= a.pos0 + q0; };
-
-  // Two LDS buffer pairs: tile kt is computed from pair (p0 + kt - kt0) & 1
-  // while tile kt + 1 loads into the other one; a wait + barrier ends each
-  // tile.
-
-  // Operands are read from LDS kAhead groups ahead of the MFMAs that use
-  // them; sched_barrier keeps the compiler from sinking each read next to its
-  // first use, where every group's LDS latency would stall the wave.
-  constexpr int kAhead = FLK_PREFILL_AHEAD;
-  constexpr int NG = DS / 4;        // S: groups of 4 k-steps (one float4 per chain)
-  constexpr int NST = kHalfKB * 4;  // PV: k-steps of 4 keys
-  // Lane group lg reads chunks 8 lg .. 8 lg + 7 (D = 128) of its key rows.
-  const int kr0 = ((half * kHalfKB) * 16 + lc) * LDK + 4 * k_chunk_pos<D, kKPerm>((DS / 4) * lg);
-  const int vr0 = ((half * kHalfKB) * 16 + 4 * lg) * D + CB * lc;
-  auto k_group = [&](const float* kt_lds_base, int g, int b) {
-    return *reinterpret_cast<const floatx4*>(kt_lds_base + b * 16 * LDK + 4 * g);
+  // Byte offsets of this lane's slot 0 + lg of its K row, V row within a plane;
+  // slot 2x + lg is that offset ^ 32x (the rows are aligned to their length).
+  const uint32_t kaddr = 16 * ((half * 32 + lc) * T::KS + (lg ^ slot_swizzle<T::KS>(lc)));
+  const uint32_t vaddr = 16 * (lc * 8 + (lg ^ slot_swizzle<8>(lc))) ^ (64 * half);
+  uint32_t kaddr_o = kaddr;
+  auto read_k = [&](uint32x4 (&f)[3], int j) {
+    const uint32x4* p = reinterpret_cast<const uint32x4*>(
+        reinterpret_cast<const char*>(bk) + (kaddr_o ^ (32 * j)));
+#pragma unroll
+    for (int k = 0; k < 3; k++) f[k] = p[k * T::kPlane];
   };
-  auto v_step = [&](const float* vt_lds_base, int st, int c4) {
-    const int b = st / 4, i = st % 4;
-    return *reinterpret_cast<const floatx4*>(vt_lds_base + (b * 16 + i) * D + 4 * (c4 ^ sw_rd));
+  // PV group n: channel block n % CB, 16-key step n / CB.
+  auto read_v = [&](uint32x4 (&f)[3], int n) {
+    const uint32x4* p = reinterpret_cast<const uint32x4*>(
+        reinterpret_cast<const char*>(bv) + (vaddr ^ (32 * (n / CB)))) + (n % CB) * 256;
+#pragma unroll
+    for (int k = 0; k < 3; k++) f[k] = p[k * T::kPlane];
   };
 
-  // The buffer of every tile is a compile-time choice (B), so that the
-  // compiler sees that the operand reads of one buffer do not depend on the
-  // loads in flight into the other and places no wait for them.
-  auto tile = [&](uint32_t kt, auto bc) {
-    constexpr int B = decltype(bc)::value;
-    float* const k_cur = B ? lb.k1 : lb.k0;
-    float* const v_cur = B ? lb.v1 : lb.v0;
-    float* const k_nxt = B ? lb.k0 : lb.k1;
-    float* const v_nxt = B ? lb.v0 : lb.v1;
+#pragma unroll 1
+  for (uint32_t kt = kt0; kt < kt1; kt++) {
     const uint32_t key0 = kt * kBK;
-    if (kt + 1 < kt1)
-      request_tile<D>(a, k_nxt, v_nxt, kvh, kt + 1, n_keys_total, toff, wave_u);
-    else if (nxt_qt >= 0)  // the next q tile's first key tile
-      request_tile<D>(a, k_nxt, v_nxt, kvh, 0, n_keys_total, toff, wave_u);
-    const float* kb = k_cur + kr0;
-    const float* vb = v_cur + vr0;
-
-    // The first K groups of this tile (in LDS since the barrier).
-    floatx4 kg[kAhead + 1][kHalfKB];
+    const uint32_t kt_1 = kt + 1 < kt1 ? kt + 1 : nxt_kt;
+    kaddr_o = kaddr;  // opaque: its xors are formed at each use
+    asm volatile("" : "+v"(kaddr_o));
+    // ---- S^T = K Q^T, V split and stored under its first half ----------------------
+    floatx16 s;
 #pragma unroll
-    for (int g = 0; g < kAhead; g++)
+    for (int i = 0; i < 16; i++) s[i] = 0.f;
+    uint32x4 f[2][3];
+    read_k(f[0], 0);
+    FLK_SCHED_FENCE();
 #pragma unroll
-      for (int b = 0; b < kHalfKB; b++) kg[g][b] = k_group(kb, g, b);
-    __builtin_amdgcn_sched_barrier(0);
-
-    // ---- S^T = K Q^T ------------------------------------------------------------
-    // Each MFMA depends on the previous one of its block's chain, so the
-    // blocks' chains are issued interleaved, step by step.
-    floatx4 sacc[kHalfKB];
+    for (int j = 0; j < NG; j++) {
+      if (j + 1 < NG) read_k(f[(j + 1) & 1], j + 1);
+      mfma_split(s, f[j & 1], qf[j]);
+      if (j < SG) {
 #pragma unroll
-    for (int b = 0; b < kHalfKB; b++) sacc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int g = 0; g < NG; g++) {
-      if (g + kAhead < NG) {
-#pragma unroll
-        for (int b = 0; b < kHalfKB; b++) kg[(g + kAhead) % (kAhead + 1)][b] = k_group(kb, g + kAhead, b);
+        for (int e = 0; e < 4; e++) stage_step<D, true>(4 * j + e, st, ld, bv, w);
       }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-#pragma unroll
-        for (int b = 0; b < kHalfKB; b++)
-          sacc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kg[g % (kAhead + 1)][b][j], qreg[4 * g + j],
-                                                         sacc[b], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
+      if (j == BG) {
+        ld.load_k(st, a, kvh, kt_1);
+        lds_barrier();
+      }
+      FLK_SCHED_FENCE();
     }
-
-    // The first V steps go out before the softmax, which does not need them.
-    floatx4 vg[kAhead + 1][CB / 4];
-#pragma unroll
-    for (int st = 0; st < kAhead; st++)
-#pragma unroll
-      for (int c4 = 0; c4 < CB / 4; c4++) vg[st][c4] = v_step(vb, st, c4);
-    __builtin_amdgcn_sched_barrier(0);
 
     // ---- online softmax of this lane's row (base 2) ----------------------------
     // Scores are base-2 already (q carries scale * log2(e)), so every weight is
     // one v_exp_f32 against the reference m_run. The reference moves only when
     // some score of the wave exceeds it by more than 8 (a factor 256): the
-    // check needs only each lane's own 8 scores, and the row's maximum across
-    // its four lane groups is formed only then (rarely after the first tile).
+    // check needs only each lane's own 16 scores, and the row's maximum across
+    // its two lanes is formed only then (rarely after the first tile).
     // Otherwise the weights are taken against the old reference -- each at
     // most 256 -- and nothing is rescaled. Tiles wholly below the causal
     // diagonal with every row live skip the mask.
-    if (!full_tile(key0)) {
+    if (!(all_rows && key0 + kBK - 1 <= a.pos0 + q0)) {
 #pragma unroll
-      for (int b = 0; b < kHalfKB; b++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const uint32_t key = key0 + (half * kHalfKB + b) * 16 + 4 * lg + i;
-          sacc[b][i] = row_ok && key <= qpos ? sacc[b][i] : -INFINITY;
-        }
+      for (int i = 0; i < 16; i++) {
+        const uint32_t key = key0 + half * 32 + 8 * (i / 4) + 4 * lg + i % 4;
+        s[i] = row_ok && key <= qpos ? s[i] : -INFINITY;
+      }
     }
-    float lmx = sacc[0][0];
+    float lmx = s[0];
 #pragma unroll
-    for (int b = 0; b < kHalfKB; b++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) lmx = fmaxf(lmx, sacc[b][i]);
+    for (int i = 1; i < 16; i++) lmx = fmaxf(lmx, s[i]);
     if (__builtin_amdgcn_ballot_w64(lmx > m_run + 8.f) != 0) {  // uniform branch
       // Only rows whose own maximum passed the threshold move their reference;
       // the others keep it and are multiplied by exactly 1, so a row's result
       // depends on its own keys only (causality holds bit for bit).
-      float mx = max_xor<16>(lmx);
-      mx = max_xor<32>(mx);
+      const float mx = max_xor<32>(lmx);
       const bool up = mx > m_run + 8.f;
       const float corr = up ? __builtin_amdgcn_exp2f(m_run - mx) : 1.f;
       l_run *= corr;
@@ -264,150 +413,173 @@ __device__ __forceinline__ void run_qtile(const PrefillArgs& a, const TileBuffer
       m_run = up ? mx : m_run;
     }
 #pragma unroll
-    for (int b = 0; b < kHalfKB; b++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float p = __builtin_amdgcn_exp2f(sacc[b][i] - m_run);
-        sacc[b][i] = p;
-        l_run += p;
-      }
-
-    // ---- O^T += V^T P^T ---------------------------------------------------------
-#pragma unroll
-    for (int st = 0; st < NST; st++) {
-      if (st + kAhead < NST) {
-#pragma unroll
-        for (int c4 = 0; c4 < CB / 4; c4++)
-          vg[(st + kAhead) % (kAhead + 1)][c4] = v_step(vb, st + kAhead, c4);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int c = 0; c < CB; c++)
-        oacc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vg[st % (kAhead + 1)][c / 4][c % 4],
-                                                       sacc[st / 4][st % 4], oacc[c], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < 16; i++) {
+      s[i] = __builtin_amdgcn_exp2f(s[i] - m_run);
+      l_run += s[i];
     }
-    wait_vm0();       // this wave's share of the next tile is in LDS
-    __syncthreads();  // every wave's; every wave is done with this tile's buffers
-  };
-  uint32_t kt = kt0;
-  if (p0 != 0 && kt < kt1) tile(kt++, std::integral_constant<int, 1>{});
-  for (; kt + 1 < kt1; kt += 2) {
-    tile(kt, std::integral_constant<int, 0>{});
-    tile(kt + 1, std::integral_constant<int, 1>{});
-  }
-  if (kt < kt1) tile(kt, std::integral_constant<int, 0>{});
+    uint32x4 pf[2][3];
+    auto split_p = [&](int e) {  // weights 2e, 2e + 1
+      uint32_t p[3];
+      split_pair(s[2 * e], s[2 * e + 1], p);
+#pragma unroll
+      for (int k = 0; k < 3; k++) pf[e / 4][k][e % 4] = p[k];
+    };
+    uint32x4 g[2][3];
+    read_v(g[0], 0);
+#pragma unroll
+    for (int e = 0; e < 4; e++) split_p(e);
 
-  l_run = sum_xor<16>(l_run);  // the row's denominator: its four lane groups
-  l_run = sum_xor<32>(l_run);
+    // ---- O^T += V^T P^T; under its first half (step 0) the weights of step 1 are
+    // split, and the next K is split and stored --------------------------------------
+#pragma unroll
+    for (int n = 0; n < NG; n++) {
+      if (n + 1 < NG) read_v(g[(n + 1) & 1], n + 1);
+      mfma_split(oacc[n % CB], g[n & 1], pf[n / CB]);
+      if (n < CB) {
+#pragma unroll
+        for (int e = 0; e < 4 / CB; e++) split_p(4 + n * (4 / CB) + e);
+      }
+      if (n < SG) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) stage_step<D, false>(4 * n + e, st, ld, bn, w);
+      }
+      if (n == BG) {
+        ld.load_v(st, a, kvh, kt_1);
+        lds_barrier();
+      }
+      FLK_SCHED_FENCE();
+    }
+    uint32x4* t = bk;
+    bk = bn;
+    bn = bv;
+    bv = t;
+  }
+
+  p.bk = bk;
+  p.bv = bv;
+  p.bn = bn;
+  QRow<D>(a, kvh, nxt_qt).fetch(p.q, a);
+  l_run = sum_xor<32>(l_run);  // the row's two lanes
   // ---- combine the two key halves of each row through LDS --------------------
-  // Lane holds channels 4*CB*lg + CB*j + c of its row. The upper waves park
-  // their acc in the last tile's K buffer and (m, l) in its V buffer; the
-  // lower waves fold them in and write the row.
-  // The last tile's buffers are free (the other pair may hold the next q
-  // tile's first key tile).
-  // o rows padded to D + FLK_PREFILL_OPAD floats: the 16 lanes of a group
-  // hold 16 different rows, which then fall in distinct bank groups.
-  constexpr int LDO = D + FLK_PREFILL_OPAD;
-  static_assert(kRows * LDO <= kBK * LDK && 2 * kRows <= kBK * D, "combine data exceeds a buffer");
-  const int buf_last = (p0 + kt1 - 1 - kt0) & 1;
-  float* m_lds = v_buf(buf_last);  // [kRows] m, then [kRows] l
-  float* o_lds = k_buf(buf_last);  // [kRows][LDO]
-  if (half == 1) {
-    float* dst = o_lds + r * LDO + 4 * CB * lg;
+  // Each half hands the other its channel blocks of the other's share (half 0
+  // finishes blocks 0 .. CB/2 - 1, half 1 the rest) and its (m, l), through the
+  // two tiles of the ring that do not hold the next item's K.
+  constexpr int HB = CB / 2;
+  static_assert(HB * 1024 + 128 <= T::kSlots, "half the exchange and (m, l) fit a tile");
+  lds_barrier();  // every wave is done with the ring
+  float2* ml_x = reinterpret_cast<float2*>(bn + HB * 1024);  // [half][kRows]
+  floatx16 mine[HB];
+#pragma unroll
+  for (int c = 0; c < HB; c++) {
+    const floatx16 give = half ? oacc[c] : oacc[HB + c];
+    mine[c] = half ? oacc[HB + c] : oacc[c];
 #pragma unroll
     for (int j = 0; j < 4; j++)
-#pragma unroll
-      for (int c4 = 0; c4 < CB / 4; c4++)
-        *reinterpret_cast<float4*>(dst + CB * j + 4 * (c4 ^ sw_wr)) =
-            make_float4(oacc[4 * c4 + 0][j], oacc[4 * c4 + 1][j], oacc[4 * c4 + 2][j],
-                        oacc[4 * c4 + 3][j]);
-    if (lg == 0) {
-      m_lds[r] = m_run;
-      m_lds[kRows + r] = l_run;
-    }
+      (half ? bn : bv)[(((wave & 3) * HB + c) * 4 + j) * 64 + lane] = __builtin_bit_cast(
+          uint32x4, make_float4(give[4 * j], give[4 * j + 1], give[4 * j + 2], give[4 * j + 3]));
   }
-  __syncthreads();
-  if (half == 1) return;
-  const float m2 = m_lds[r], l2 = m_lds[kRows + r];
-  const float M = fmaxf(m_run, m2);
+  if (lg == 0) ml_x[half * kRows + r] = make_float2(m_run, l_run);
+  if (threadIdx.x == 0) *s_bad = 0;
+  lds_barrier();
+  const float2 ml2 = ml_x[(1 - half) * kRows + r];
+  const float M = fmaxf(m_run, ml2.x);
   // A half that saw no key of this row still holds the initial reference
-  // (-1e30, l = 0): its weight exp2(-1e30 - M) is 0.
+  // (-1e30, l = 0): its weight exp2(-1e30 - M) is 0. A row with no key in the
+  // item at all has both at the initial reference and sums of 0.
   const float w1 = __builtin_amdgcn_exp2f(m_run - M);
-  const float w2 = __builtin_amdgcn_exp2f(m2 - M);
-  const float L = l_run * w1 + l2 * w2;
-  const float* o2 = o_lds + r * LDO + 4 * CB * lg;
+  const float w2 = __builtin_amdgcn_exp2f(ml2.x - M);
+  const float L = l_run * w1 + ml2.y * w2;
   float* dst;
   if (final) {
-    if (!row_ok) return;
-    dst = a.o + ((size_t)qi * a.n_heads + h) * D + 4 * CB * lg;
+    dst = a.o + row.offset(a);
   } else {
-    dst = a.part_acc + (slot * kRows + r) * D + 4 * CB * lg;
-    if (lg == 0) a.part_ml[slot * kRows + r] = make_float2(M, L);
+    dst = a.part_acc + (slot * kRows + r) * D;
+    if (lg == 0 && half == 0) a.part_ml[slot * kRows + r] = make_float2(M, L);
   }
+  bool bad = false;
+  auto redo = [](float x) { return !(fabsf(x) >= kTinyOutput) && x != 0.f; };
 #pragma unroll
-  for (int j = 0; j < 4; j++)
+  for (int c = 0; c < HB; c++)
 #pragma unroll
-    for (int c4 = 0; c4 < CB / 4; c4++) {
-      const float4 p = *reinterpret_cast<const float4*>(o2 + CB * j + 4 * (c4 ^ sw_wr));
-      float4 v = make_float4(oacc[4 * c4 + 0][j] * w1 + p.x * w2,
-                             oacc[4 * c4 + 1][j] * w1 + p.y * w2,
-                             oacc[4 * c4 + 2][j] * w1 + p.z * w2,
-                             oacc[4 * c4 + 3][j] * w1 + p.w * w2);
+    for (int j = 0; j < 4; j++) {
+      const float4 x = __builtin_bit_cast(
+          float4, (half ? bv : bn)[(((wave & 3) * HB + c) * 4 + j) * 64 + lane]);
+      float4 v = make_float4(mine[c][4 * j] * w1 + x.x * w2, mine[c][4 * j + 1] * w1 + x.y * w2,
+                             mine[c][4 * j + 2] * w1 + x.z * w2,
+                             mine[c][4 * j + 3] * w1 + x.w * w2);
       if (final) v = make_float4(v.x / L, v.y / L, v.z / L, v.w / L);
-      *reinterpret_cast<float4*>(dst + CB * j + 4 * (c4 ^ sw_wr)) = v;
+      bad |= redo(v.x) || redo(v.y) || redo(v.z) || redo(v.w);
+      if (row_ok || !final)
+        *reinterpret_cast<float4*>(dst + 32 * (HB * half + c) + 8 * j + 4 * lg) = v;
     }
+  bad |= !final && L != L;
+  if (row_ok && bad) *s_bad = 1;
+  // Every wave is done with the exchange (the next item's V goes there), and its
+  // stores are out before item_f32's.
+  __syncthreads();
+  if (*s_bad) {
+    item_f32<D>(a, kvh, qt, kt0, kt1, final, slot);
+    __syncthreads();
+  }
 }
 
 template <int D>
-__global__ __launch_bounds__(kPThreads) void prefill_kernel(PrefillArgs a) {
-  __shared__ __attribute__((aligned(16))) float k_lds0[kBK * (D + 4)];
-  __shared__ __attribute__((aligned(16))) float k_lds1[kBK * (D + 4)];
-  __shared__ __attribute__((aligned(16))) float v_lds0[kBK * D];
-  __shared__ __attribute__((aligned(16))) float v_lds1[kBK * D];
-  const TileBuffers lb{k_lds0, k_lds1, v_lds0, v_lds1};
+__global__ __launch_bounds__(kPThreads, 2) void prefill_kernel(PrefillArgs a, PrefillTable tab) {
+  __shared__ uint32x4 lds[3 * SplitTile<D>::kSlots];
+  __shared__ int s_bad;
   const uint32_t kvh = blockIdx.x % a.n_kv_heads;
   const uint32_t w = blockIdx.x / a.n_kv_heads;
-  float4 qraw[D / 16];
-  TileOffsets<D> toff;
-  tile_offsets<D>(toff, a.n_kv_heads * D * 4, threadIdx.x >> 6, threadIdx.x & 63);
-  if (a.paired) {
-    const uint32_t qt_hi = a.n_qtiles - 1 - w;
-    const uint32_t n_hi = qtile_kt(qt_hi, a.q_per_tile, a.n_queries, a.pos0);
-    run_qtile<D>(a, lb, kvh, qt_hi, 0, n_hi, true, 0, qraw, toff, 0, false,
-                 w < qt_hi ? (int)w : -1);
-    if (w < qt_hi)
-      run_qtile<D>(a, lb, kvh, w, 0, qtile_kt(w, a.q_per_tile, a.n_queries, a.pos0),
-                   true, 0, qraw, toff, n_hi & 1, true, -1);
-    return;
+  const TileLoader<D> ld(a.n_kv_heads * D * 4);
+  const PrefillStart s0 = tab.start[w], s1 = tab.start[w + 1];
+  uint32_t seq = s0.seq, kt0 = s0.kt;
+  auto live = [&](uint32_t x, uint32_t kt) { return x < s1.seq || (x == s1.seq && kt < s1.kt); };
+  if (!live(seq, kt0)) return;  // uniform
+  Pipe<D> p;
+  p.bk = lds;
+  p.bv = lds + SplitTile<D>::kSlots;
+  p.bn = lds + 2 * SplitTile<D>::kSlots;
+  ld.load_k(p.st, a, kvh, kt0);
+  QRow<D>(a, kvh, prefill_seq_qt(seq, a.n_qtiles)).fetch(p.q, a);
+  ld.load_v(p.st, a, kvh, kt0);
+  uint32x4 t[3];
+#pragma unroll
+  for (int n = 0; n < 4 * SplitTile<D>::KP; n++) stage_step<D, false>(n, p.st, ld, p.bk, t);
+  while (live(seq, kt0)) {
+    const uint32_t qt = prefill_seq_qt(seq, a.n_qtiles);
+    const uint32_t n_kt = qtile_kt(qt, a.q_per_tile, a.n_queries, a.pos0);
+    const uint32_t kt1 = seq == s1.seq ? s1.kt : n_kt;
+    // A workgroup's first piece of a cut q tile has slot 2w, its last 2w + 1.
+    const size_t slot = (size_t)(2 * w + (seq != s0.seq ? 1 : 0)) * a.n_kv_heads + kvh;
+    const bool more = live(seq + 1, 0);
+    run_item<D>(a, p, &s_bad, kvh, qt, kt0, kt1, kt0 == 0 && kt1 == n_kt, slot, ld,
+                more ? prefill_seq_qt(seq + 1, a.n_qtiles) : qt, more ? 0 : kt0);
+    seq++;
+    kt0 = 0;
   }
-  const uint32_t qt = a.n_qtiles - 1 - w / a.max_splits;  // heaviest q tile first
-  const uint32_t split = w % a.max_splits;
-  const uint32_t n_kt = qtile_kt(qt, a.q_per_tile, a.n_queries, a.pos0);
-  const uint32_t ns = (n_kt + a.kt_per_split - 1) / a.kt_per_split;
-  if (split >= ns) return;  // uniform per workgroup
-  const uint32_t kt0 = split * n_kt / ns;
-  const uint32_t kt1 = (split + 1) * n_kt / ns;
-  const size_t slot = ((size_t)qt * a.max_splits + split) * a.n_kv_heads + kvh;
-  run_qtile<D>(a, lb, kvh, qt, kt0, kt1, ns == 1, slot, qraw, toff, 0, false, -1);
 }
 
-// One workgroup per (kv head, q tile, 256 / (D/4) rows); D/4 lanes per row,
-// each owning a float4 of channels. Combines the splits of a multi-split q
-// tile with log-sum-exp weights in one pass: the splits go in rounds of
-// kPMergeBatch whose loads are all issued first (indices past the last split
-// reload it and get weight 0, so every load is unconditional), then folded
-// against a running maximum. Single-split tiles exit.
+// One workgroup per (kv head, workgroup w of prefill_kernel, 256 / (D/4)
+// rows); D/4 lanes per row, each owning a float4 of channels. If a cut q tile
+// starts in w, combines its pieces (w's last or only one, then the first of w +
+// 1, w + 2, ... until the tile ends) with log-sum-exp weights in one pass: the
+// pieces go in rounds of kPMergeBatch whose loads are all issued first (indices
+// past the last piece reload it and get weight 0, so every load is
+// unconditional), then folded against a running maximum.
 constexpr int kPMergeBatch = 8;
 template <int D>
-__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, PrefillTable tab) {
   constexpr int LPR = D / 4;
   constexpr int RPB = 256 / LPR;   // rows per block
   const uint32_t kvh = blockIdx.x;
-  const uint32_t qt = blockIdx.y;
-  const uint32_t n_kt = qtile_kt(qt, a.q_per_tile, a.n_queries, a.pos0);
-  const uint32_t ns = (n_kt + a.kt_per_split - 1) / a.kt_per_split;
-  if (ns == 1) return;
+  const uint32_t w = blockIdx.y;
+  const uint32_t seq = tab.start[w + 1].seq;
+  const PrefillStart s0 = tab.start[w];
+  // Cut at the end of w, and started in w.
+  if (tab.start[w + 1].kt == 0 || (s0.seq == seq && s0.kt != 0)) return;
+  const uint32_t first = 2 * w + (s0.seq != seq ? 1 : 0);
+  uint32_t ns = 2;
+  while (tab.start[w + ns].seq == seq && tab.start[w + ns].kt != 0) ns++;
+  const uint32_t qt = prefill_seq_qt(seq, a.n_qtiles);
   const uint32_t r = blockIdx.z * RPB + threadIdx.x / LPR;
   const int c = threadIdx.x % LPR;
   const uint32_t qi = qt * a.q_per_tile + r / a.group;
@@ -415,22 +587,25 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   const uint32_t h = kvh * a.group + r % a.group;
   float M = -INFINITY, L = 0.f;
   float4 A = make_float4(0.f, 0.f, 0.f, 0.f);
-  for (uint32_t s0 = 0; s0 < ns; s0 += kPMergeBatch) {
+  for (uint32_t p0 = 0; p0 < ns; p0 += kPMergeBatch) {
     float2 ml[kPMergeBatch];
     float4 pa[kPMergeBatch];
 #pragma unroll
     for (int i = 0; i < kPMergeBatch; i++) {
-      const uint32_t sp = min(s0 + i, ns - 1);
-      const size_t slot = ((size_t)qt * a.max_splits + sp) * a.n_kv_heads + kvh;
+      const uint32_t sp = min(p0 + i, ns - 1);
+      const size_t slot = (size_t)(sp == 0 ? first : 2 * (w + sp)) * a.n_kv_heads + kvh;
       ml[i] = a.part_ml[slot * kRows + r];
       pa[i] = reinterpret_cast<const float4*>(a.part_acc + (slot * kRows + r) * D)[c];
     }
 #pragma unroll
     for (int i = 0; i < kPMergeBatch; i++)
-      if (s0 + i >= ns) ml[i].x = -INFINITY;  // a reloaded split: weight 0
+      if (p0 + i >= ns) {  // a reloaded piece: weight 0
+        ml[i].x = -INFINITY;
+        pa[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
     float mx = M;
 #pragma unroll
-    for (int i = 0; i < kPMergeBatch; i++) mx = fmaxf(mx, ml[i].x);  // finite: split s0 is live
+    for (int i = 0; i < kPMergeBatch; i++) mx = fmaxf(mx, ml[i].x);  // piece p0's is no -inf
     const float wo = __builtin_amdgcn_exp2f(M - mx);  // m is in log2 units; exp2(-inf) = 0
     L *= wo;
     A.x *= wo;
@@ -439,12 +614,12 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     A.w *= wo;
 #pragma unroll
     for (int i = 0; i < kPMergeBatch; i++) {
-      const float w = __builtin_amdgcn_exp2f(ml[i].x - mx);
-      L = fmaf(ml[i].y, w, L);
-      A.x = fmaf(pa[i].x, w, A.x);
-      A.y = fmaf(pa[i].y, w, A.y);
-      A.z = fmaf(pa[i].z, w, A.z);
-      A.w = fmaf(pa[i].w, w, A.w);
+      const float wt = __builtin_amdgcn_exp2f(ml[i].x - mx);
+      L = fmaf(ml[i].y, wt, L);
+      A.x = fmaf(pa[i].x, wt, A.x);
+      A.y = fmaf(pa[i].y, wt, A.y);
+      A.z = fmaf(pa[i].z, wt, A.z);
+      A.w = fmaf(pa[i].w, wt, A.w);
     }
     M = mx;
   }
@@ -453,89 +628,124 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
 }
 
 // ------------------------------------------------------------------ plan ----
+static uint64_t prefill_max_wg(uint32_t n_kv_heads) {
+  return n_kv_heads < kMaxWG ? kMaxWG / n_kv_heads : 1;
+}
+
+// Estimated time (us) of the f32 kernel under its plan: 1-tile items cost 5 +
+// 4.4 (head_dim 64: 3.5 + 2.5), a merge 5; more workgroups than CUs run in rounds.
+static double small_us(const f32::PrefillPlan& p, uint32_t n_kv_heads, uint32_t head_dim,
+                       uint32_t n_queries, uint32_t pos0) {
+  uint64_t wg = 0, run = 0;
+  if (p.paired) {
+    wg = p.work_per_kvh;
+    run = qtile_kt(p.n_qtiles - 1, p.q_per_tile, n_queries, pos0) +
+          qtile_kt(0, p.q_per_tile, n_queries, pos0);
+  } else {
+    run = p.ktiles_per_split;
+    for (uint32_t qt = 0; qt < p.n_qtiles; qt++)
+      wg += (qtile_kt(qt, p.q_per_tile, n_queries, pos0) + run - 1) / run;
+    const uint64_t heaviest = qtile_kt(p.n_qtiles - 1, p.q_per_tile, n_queries, pos0);
+    if (run > heaviest) run = heaviest;
+  }
+  const double rounds = (double)((wg * n_kv_heads + kMaxWG - 1) / kMaxWG);
+  const double tiles = rounds * run;
+  return (head_dim == 128 ? 5.0 + 4.4 * tiles : 3.5 + 2.5 * tiles) + (p.max_splits > 1 ? 5.0 : 0.0);
+}
+
+// A kv head's q tiles either stay whole, one workgroup each (or, with more of
+// them than workgroups, equal runs of them), or are cut into equal runs of key
+// tiles, which costs a merge: the run with the least estimated time, from (us,
+// measured) 8 + 5 per key tile of the longest run (head_dim 64: 5 + 2.8), and for
+// the merge 5 + 1.3 per 8 pieces of a q tile. Calls that the f32 kernel is
+// estimated to finish within 1.3 times that take it (over 155 shapes of 1 to 300
+// heads, 9 to 1024 tokens and 0 to 16000 keys before them no call is then slower
+// than under the f32 kernel alone; with 1.1, three were): with 16 / 8 heads of 128,
+// us, f32 kernel against this one, 64 tokens at 2000 22.6 / 36.6, 300 at 448 27 /
+// 33, 512 at 448 52 / 38, 300 at 2000 93 / 51, 200 at 16000 403 / 168.
 PrefillPlan prefill_plan(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
                          uint32_t n_queries, uint32_t pos0) {
   PrefillPlan p{};
-  const uint32_t group = n_heads / n_kv_heads;
-  p.rows_per_tile = kRows;
-  p.q_per_tile = kRows / group;
+  p.q_per_tile = kRows / (n_heads / n_kv_heads);
   p.n_qtiles = (n_queries + p.q_per_tile - 1) / p.q_per_tile;
-  const uint32_t pairs = (p.n_qtiles + 1) / 2;
-  if ((uint64_t)pairs * n_kv_heads >= kMinPairedWG) {
-    p.paired = 1;
-    p.work_per_kvh = pairs;
-    p.ktiles_per_split = 0;
-    p.max_splits = 1;
-    p.partial_slots = 0;
-    return p;
+  for (uint32_t qt = 0; qt < p.n_qtiles; qt++)
+    p.key_tiles += qtile_kt(qt, p.q_per_tile, n_queries, pos0);
+  const uint64_t most = prefill_max_wg(n_kv_heads);
+  const uint64_t max_kt = qtile_kt(p.n_qtiles - 1, p.q_per_tile, n_queries, pos0);
+  const uint64_t least = (p.key_tiles + most - 1) / most;
+  const uint64_t rounds = (n_kv_heads + kMaxWG - 1) / kMaxWG;
+  const double t0 = head_dim == 128 ? 8.0 : 5.0, t1 = head_dim == 128 ? 5.0 : 2.8;
+  // Runs of whole q tiles end up to a q tile late.
+  const uint64_t whole =
+      p.n_qtiles <= most ? max_kt : (least > max_kt ? least : max_kt) + max_kt / 2;
+  double best = t0 + t1 * rounds * whole;
+  p.wg_per_kvh = (uint32_t)(p.n_qtiles < most ? p.n_qtiles : most);
+  for (uint64_t run = least; run <= 4 * least && run < whole; run++) {
+    const uint64_t pieces = (max_kt + run - 1) / run + 1;
+    const double t = t0 + t1 * rounds * run + 5.0 + 1.3 * ((pieces + 7) / 8);
+    if (t < best) {
+      best = t;
+      p.cut = true;
+      p.wg_per_kvh = (uint32_t)((p.key_tiles + run - 1) / run);
+    }
   }
-  uint64_t total = 0;
-  for (uint32_t qt = 0; qt < p.n_qtiles; qt++) total += qtile_kt(qt, p.q_per_tile, n_queries, pos0);
-  total *= n_kv_heads;
-  uint64_t ch = (total + kTargetSplitWG - 1) / kTargetSplitWG;
-  if (ch < kMinKtPerSplit) ch = kMinKtPerSplit;
-  const uint32_t max_kt = qtile_kt(p.n_qtiles - 1, p.q_per_tile, n_queries, pos0);
-  const uint64_t ms = (max_kt + ch - 1) / ch;
-  p.paired = 0;
-  p.ktiles_per_split = (uint32_t)ch;
-  p.max_splits = (uint32_t)ms;
-  p.work_per_kvh = p.n_qtiles * p.max_splits;
-  p.partial_slots = ms > 1 ? (uint64_t)p.n_qtiles * ms * n_kv_heads : 0;
+  p.partial_slots = p.cut ? 2ull * p.wg_per_kvh * n_kv_heads : 0;
+  p.small = f32::prefill_plan(n_heads, n_kv_heads, head_dim, n_queries, pos0);
+  p.use_small = small_us(p.small, n_kv_heads, head_dim, n_queries, pos0) < 1.3 * best;
   return p;
 }
 
+static uint64_t split_ws_bytes(uint64_t slots, uint32_t head_dim) {
+  if (slots == 0) return 0;
+  return ws_align(slots * kRows * sizeof(float2)) + slots * kRows * head_dim * sizeof(float);
+}
+
 uint64_t prefill_ws_bytes(const PrefillPlan& p, uint32_t head_dim) {
-  if (p.partial_slots == 0) return 0;
-  return ws_align(p.partial_slots * kRows * sizeof(float2)) +
-         p.partial_slots * kRows * head_dim * sizeof(float);
+  return p.use_small ? f32::prefill_ws_bytes(p.small, head_dim)
+                     : split_ws_bytes(p.partial_slots, head_dim);
 }
 
 // Upper bound over every plan with n_queries <= max_queries and pos0 +
-// n_queries <= max_keys. Only split plans have partials, and only while
-// ceil(n_qtiles / 2) * n_kv_heads < kMinPairedWG. In a split plan the last q
-// tile alone gives total >= n_kv_heads * max_kt key tiles, so ch >= n_kv_heads
-// * max_kt / kTargetSplitWG and ms = ceil(max_kt / ch) <= ceil(kTargetSplitWG /
-// n_kv_heads); also ms <= ceil(max_kt / kMinKtPerSplit) with max_kt <=
-// ceil(max_keys / kBK).
+// n_queries <= max_keys: the last max_queries of max_keys positions have the
+// most key tiles, and a cut plan has at most one workgroup for each.
 uint64_t prefill_ws_bound(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
                           uint32_t max_queries, uint32_t max_keys) {
-  const uint32_t qpt = kRows / (n_heads / n_kv_heads);
-  const uint64_t max_qt = (max_queries + qpt - 1) / qpt;
-  uint64_t nqt = 0;  // most q tiles a split plan can have
-  for (uint64_t t = 1; t <= max_qt && (t + 1) / 2 * n_kv_heads < kMinPairedWG; t++) nqt = t;
-  if (nqt == 0) return 0;
-  const uint64_t max_kt = ((uint64_t)max_keys + kBK - 1) / kBK;
-  const uint64_t by_wg = (kTargetSplitWG + n_kv_heads - 1) / n_kv_heads;
-  const uint64_t by_kt = (max_kt + kMinKtPerSplit - 1) / kMinKtPerSplit;
-  const uint64_t ms = by_wg < by_kt ? by_wg : by_kt;
-  if (ms <= 1) return 0;
-  PrefillPlan p{};
-  p.partial_slots = nqt * ms * n_kv_heads;
-  return prefill_ws_bytes(p, head_dim);
+  const PrefillPlan p =
+      prefill_plan(n_heads, n_kv_heads, head_dim, max_queries, max_keys - max_queries);
+  const uint64_t most = prefill_max_wg(n_kv_heads);
+  const uint64_t wg = p.key_tiles < most ? p.key_tiles : most;
+  const uint64_t split = split_ws_bytes(wg > 1 ? 2 * wg * n_kv_heads : 0, head_dim);
+  const uint64_t small =
+      f32::prefill_ws_bound(n_heads, n_kv_heads, head_dim, max_queries, max_keys);
+  return split > small ? split : small;
 }
 
 template <int D>
-static hipError_t launch_prefill_d(const PrefillArgs& a, const PrefillPlan& p, hipStream_t st) {
-  const dim3 grid(a.n_kv_heads * p.work_per_kvh);
-  hipLaunchKernelGGL(prefill_kernel<D>, grid, dim3(kPThreads), 0, st, a);
+static hipError_t launch_prefill_d(const PrefillArgs& a, const PrefillTable& tab, bool cut, hipStream_t st) {
+  const dim3 grid(a.n_kv_heads * a.wg_per_kvh);
+  hipLaunchKernelGGL(prefill_kernel<D>, grid, dim3(kPThreads), 0, st, a, tab);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || p.paired || p.max_splits <= 1) return e;
+  if (e != hipSuccess || !cut) return e;
   constexpr int RPB = 256 / (D / 4);
-  const dim3 mgrid(a.n_kv_heads, p.n_qtiles, kRows / RPB);
-  hipLaunchKernelGGL(prefill_merge_kernel<D>, mgrid, dim3(256), 0, st, a);
+  const dim3 mgrid(a.n_kv_heads, a.wg_per_kvh - 1, kRows / RPB);
+  hipLaunchKernelGGL(prefill_merge_kernel<D>, mgrid, dim3(256), 0, st, a, tab);
   return hipGetLastError();
 }
 
 hipError_t launch_prefill(const float* q, const float* kcache, const float* vcache, float* o,
                           uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
-                          uint32_t n_queries, uint32_t pos0, void* ws, hipStream_t st) {
-  const PrefillPlan p = prefill_plan(n_heads, n_kv_heads, head_dim, n_queries, pos0);
+                          uint32_t n_queries, uint32_t pos0, const PrefillPlan& p, void* ws,
+                          hipStream_t st) {
+  if (p.use_small)
+    return f32::launch_prefill(q, kcache, vcache, o, n_heads, n_kv_heads, head_dim, n_queries,
+                               pos0, p.small, ws, st);
   PrefillArgs a{};
+  PrefillTable tab;
   a.q = q;
   a.kcache = kcache;
   a.vcache = vcache;
   a.o = o;
-  if (p.partial_slots > 0) {
+  if (p.cut) {
     char* w = static_cast<char*>(ws);
     a.part_ml = reinterpret_cast<float2*>(w);
     a.part_acc = reinterpret_cast<float*>(w + ws_align(p.partial_slots * kRows * sizeof(float2)));
@@ -547,13 +757,32 @@ hipError_t launch_prefill(const float* q, const float* kcache, const float* vcac
   a.pos0 = pos0;
   a.q_per_tile = p.q_per_tile;
   a.n_qtiles = p.n_qtiles;
-  a.paired = p.paired;
-  a.work_per_kvh = p.work_per_kvh;
-  a.kt_per_split = p.ktiles_per_split;
-  a.max_splits = p.max_splits;
+  a.wg_per_kvh = p.wg_per_kvh;
   a.scale_log2e = (float)(1.4426950408889634 / sqrt((double)head_dim));
-  if (head_dim == 128) return launch_prefill_d<128>(a, p, st);
-  return launch_prefill_d<64>(a, p, st);
+  const bool one_each = !p.cut && p.n_qtiles == p.wg_per_kvh;
+  bool pieces = false;
+  uint64_t before = 0;  // key tiles before q tile `seq` of the order
+  uint32_t seq = 0;
+  for (uint32_t x = 0; x <= p.wg_per_kvh; x++) {
+    if (one_each) {
+      tab.start[x] = PrefillStart{x, 0};
+      continue;
+    }
+    // Workgroup x starts at key tile x * key_tiles / wg_per_kvh of the order, or
+    // with the q tile that holds it.
+    const uint64_t at = x * p.key_tiles / p.wg_per_kvh;
+    while (seq < p.n_qtiles) {
+      const uint32_t n =
+          qtile_kt(prefill_seq_qt(seq, p.n_qtiles), p.q_per_tile, n_queries, pos0);
+      if (at < before + n) break;
+      before += n;
+      seq++;
+    }
+    tab.start[x] = PrefillStart{seq, p.cut ? (uint32_t)(at - before) : 0};
+    pieces |= tab.start[x].kt != 0;
+  }
+  if (head_dim == 128) return launch_prefill_d<128>(a, tab, pieces, st);
+  return launch_prefill_d<64>(a, tab, pieces, st);
 }
 
 }  // namespace flk

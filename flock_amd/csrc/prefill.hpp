@@ -1,152 +1,128 @@
-// Prefill kernel pieces: arguments, key-tile counts, and the loads that bring
-// one 64-key K/V tile from HBM straight into LDS.
+// Prefill kernel pieces: arguments, the schedule of key tiles over workgroups,
+// the three-part bf16 split and the layout of split K/V tiles in LDS.
 #pragma once
 
 #include "common.hpp"
 
 namespace flk {
 
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-
-constexpr int kRows = 64;    // query-head rows per q tile
-constexpr int kBK = 64;      // keys per tile
+constexpr int kRows = 128;      // query-head rows per q tile (4 blocks of 32)
+constexpr int kBK = 64;         // keys per tile (2 halves of 32)
 constexpr int kPThreads = 512;  // 8 waves: 4 row blocks x 2 key halves
-constexpr int kHalfKB = 2;      // 16-key blocks per wave per tile
-constexpr uint32_t kMinPairedWG = 192;    // paired mode when it yields this many
-constexpr uint32_t kTargetSplitWG = 256;  // split mode aims at one workgroup per CU
-constexpr uint32_t kMinKtPerSplit = 2;
-#ifndef FLK_PREFILL_OPAD
-#define FLK_PREFILL_OPAD 4  // padding of the combine's o rows in LDS (floats)
-#endif
-#ifndef FLK_PREFILL_AHEAD
-#define FLK_PREFILL_AHEAD 1  // operand groups read from LDS ahead of their MFMAs
-#endif
-#ifndef FLK_PREFILL_KPERM
-#define FLK_PREFILL_KPERM 1  // K rows stored with chunks 8..15 and 16..23 swapped (D = 128)
-#endif
-constexpr bool kKPerm = FLK_PREFILL_KPERM != 0;
+constexpr uint32_t kMaxWG = 256;      // one workgroup per CU
+
+// Where workgroup w of a kv head starts: key tile kt of the seq-th q tile (in
+// the order of prefill_seq_qt). Workgroup w runs from start[w] up to start[w + 1].
+struct PrefillStart {
+  uint32_t seq, kt;
+};
 
 struct PrefillArgs {
   const float* q;
   const float* kcache;
   const float* vcache;
   float* o;
-  float2* part_ml;   // [slot][kRows]
+  float2* part_ml;   // [slot][kRows], slot = (2 w + last piece?) * n_kv_heads + kv head
   float* part_acc;   // [slot][kRows][D]
   uint32_t n_heads, n_kv_heads, group;
   uint32_t n_queries, pos0;
   uint32_t q_per_tile, n_qtiles;
-  uint32_t paired, work_per_kvh;
-  uint32_t kt_per_split, max_splits;
+  uint32_t wg_per_kvh;
   float scale_log2e;  // fr(1/sqrt(d) * log2(e)): scores in base-2 units
+};
+
+struct PrefillTable {
+  PrefillStart start[kMaxWG + 1];
 };
 
 __host__ __device__ __forceinline__ uint32_t qtile_kt(uint32_t qt, uint32_t q_per_tile,
                                                       uint32_t n_queries, uint32_t pos0) {
   const uint32_t q_end = (qt + 1) * q_per_tile < n_queries ? (qt + 1) * q_per_tile : n_queries;
-  return (pos0 + q_end + kBK - 1) / kBK;
+  return (uint32_t)(((uint64_t)pos0 + q_end + kBK - 1) / kBK);
+}
+
+// The q tiles in the order the workgroups take them: the heaviest, the
+// lightest, the next heaviest, ... so that any stretch of a prompt's causal
+// work cut out of the order holds about as many q tiles as any other.
+__host__ __device__ __forceinline__ uint32_t prefill_seq_qt(uint32_t seq, uint32_t n_qtiles) {
+  return seq & 1 ? seq >> 1 : n_qtiles - 1 - (seq >> 1);
 }
 
 // gfx9 buffer-descriptor word 3 for untyped 32-bit-element loads.
 constexpr int kBufferWord3 = 0x00020000;
 
-// Position of float4 chunk c within a K row in LDS (an involution). PERM
-// (head_dim 128) swaps chunks 8..15 with 16..23, so that 32 lanes reading 16
-// key rows at chunks g and 8 + g (or 16 + g and 24 + g) hit distinct banks of
-// the 128.
-template <int D, bool PERM>
-__device__ __forceinline__ int k_chunk_pos(int c) {
-  if constexpr (PERM && D == 128) return (c >= 8 && c < 24) ? (c ^ 24) : c;
-  return c;
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef uint32_t uint32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t uint32x2 __attribute__((ext_vector_type(2)));
+
+// ---- f32 as three bf16 -------------------------------------------------------
+// x = s[0] + s[1] + s[2] exactly (each part takes the next 8 of the 24
+// significand bits, rounded to nearest; both differences are exact). Parts of
+// two values packed as the matrix operands want them.
+__device__ __forceinline__ uint32_t bf16_pack(float a, float b) {
+  const floatx2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t (&s)[3]) {
+  s[0] = bf16_pack(a, b);
+  a -= __builtin_bit_cast(float, s[0] << 16);
+  b -= __builtin_bit_cast(float, s[0] & 0xffff0000u);
+  s[1] = bf16_pack(a, b);
+  a -= __builtin_bit_cast(float, s[1] << 16);
+  b -= __builtin_bit_cast(float, s[1] & 0xffff0000u);
+  s[2] = bf16_pack(a, b);
 }
 
-// ---- key tiles straight into LDS -------------------------------------------
-// A key tile goes from HBM to LDS with buffer_load_dwordx4 ... lds: each such
-// wave instruction writes 64 consecutive 16-byte LDS slots, lane l into slot
-// l, from the address lane l names, so the LDS layout is set by which float4
-// of the tile each lane fetches. The K tile is kBK rows of D + 4 floats (D/4 +
-// 1 slots; the last slot of a row is padding, fetched from an offset past the
-// descriptor's end, which writes zeros), its chunks placed by k_chunk_pos; the
-// V tile is kBK rows of D floats in natural order. Wave w issues the wave
-// instructions w, w + 8, ...: D/4 + 1 of them for K, D/4 for V. The descriptor
-// covers the tile's live rows only, so rows past the last key arrive as zeros
-// too. The loads count on vmcnt: a wait for vmcnt(0) and then a barrier make
-// a tile visible to every wave.
-constexpr uint32_t kPastEnd = 0x7ffffff0u;  // an offset beyond every descriptor
+// acc += sum over k of a[k] b[k] with both operands in three parts: the six
+// products of at least 2^-18 of the whole, smallest first. The three left out
+// are at most 2^-26 of |a| |b| together.
+__device__ __forceinline__ void mfma_split(floatx16& acc, const uint32x4 (&a)[3],
+                                           const uint32x4 (&b)[3]) {
+  auto mul = [&](int i, int j) {
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[i]),
+                                                  __builtin_bit_cast(bf16x8, b[j]), acc, 0, 0, 0);
+  };
+  mul(2, 0);
+  mul(0, 2);
+  mul(1, 1);
+  mul(1, 0);
+  mul(0, 1);
+  mul(0, 0);
+}
+
+// ---- split tiles in LDS --------------------------------------------------------
+// A tile is three planes (one per part) of 16-byte slots, each slot 8 bf16: one
+// lane's share of a 16-deep matrix operand.
+//   K: [64 keys][D / 8 slots]; slot c of a key holds dims 4c .. 4c + 3 and D/2 +
+//      4c .. D/2 + 4c + 3 (so that the lanes that load a key's row read it as
+//      contiguous float4s; q is permuted alike, and a dot product has no order).
+//   V: [D channels][8 slots]; slot 2s + g of a channel holds keys 16s + 4g + {0
+//      .. 3} and 16s + 8 + 4g + {0 .. 3}: the order in which lane half g holds
+//      its scores of 16-key step s after S^T = K Q^T.
+// The slot number is xored with bits of the row, so that any 8 (and 16, and 32)
+// neighbouring lanes that read one slot of consecutive rows, or write a row, or
+// write one slot of every other row, hit distinct banks.
+template <int NS>
+__device__ __forceinline__ int slot_swizzle(int row) {
+  if constexpr (NS == 16) return (row & 15) ^ ((row >> 4) & 1);
+  return (row & 7) ^ ((row >> 3) & 1) ^ (((row >> 4) & 1) << 1);
+}
 
 template <int D>
-struct TileOffsets {
-  static constexpr int KS = D / 4 + 1;         // slots of a K row
-  static constexpr int KW = kBK * KS / 64;     // K wave instructions per tile
-  static constexpr int VW = kBK * D / 4 / 64;  // V wave instructions per tile
-  static constexpr int KI = (KW + 7) / 8;      // per wave (the last one for wave 0 only)
-  static constexpr int VI = VW / 8;            // per wave
-  static_assert(KW == 8 * (KI - 1) + 1 && VW == 8 * VI, "wave instructions per tile");
-  uint32_t k[KI];
-  uint32_t v[VI];
+struct SplitTile {
+  static constexpr int KS = D / 8;              // slots of a key
+  static constexpr int kPlane = kBK * KS;       // slots of a plane (K and V alike)
+  static constexpr int kSlots = 3 * kPlane;
+  static constexpr int KP = kPlane / kPThreads;  // K slots (and V slots) a thread stages
 };
 
-// This lane's byte offsets within a tile's descriptor: the same for every
-// tile of every q tile.
-template <int D>
-__device__ __forceinline__ void tile_offsets(TileOffsets<D>& t, uint32_t row_bytes, int wave,
-                                             int lane) {
-  using T = TileOffsets<D>;
-#pragma unroll
-  for (int i = 0; i < T::KI; i++) {
-    const int s = 64 * (wave + 8 * i) + lane;
-    const int row = s / T::KS, pos = s % T::KS;
-    t.k[i] = pos < D / 4 && row < kBK ? row * row_bytes + 16 * k_chunk_pos<D, kKPerm>(pos)
-                                      : kPastEnd;
-  }
-#pragma unroll
-  for (int i = 0; i < T::VI; i++) {
-    const int s = 64 * (wave + 8 * i) + lane;
-    t.v[i] = (s / (D / 4)) * row_bytes + 16 * (s % (D / 4));
-  }
+// s_barrier once this wave's LDS operations are done; unlike __syncthreads it
+// leaves loads from memory in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
-
-#define FLK_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
-
-// Requests key tile kt of kv head kvh into one K and one V buffer. `wave`
-// must be wave-uniform: it selects the LDS addresses.
-template <int D>
-__device__ __forceinline__ void request_tile(const PrefillArgs& a, float* k_buf, float* v_buf,
-                                             uint32_t kvh, uint32_t kt, uint32_t n_keys_total,
-                                             const TileOffsets<D>& t, int wave) {
-  using T = TileOffsets<D>;
-  const uint32_t key0 = kt * kBK;
-  const uint32_t rows = min(n_keys_total - key0, (uint32_t)kBK);
-  const uint32_t row_bytes = a.n_kv_heads * D * 4;
-  const size_t base = (size_t)key0 * row_bytes + (size_t)kvh * D * 4;
-  const uint32_t n_bytes = (rows - 1) * row_bytes + D * 4;
-  const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char*>(reinterpret_cast<const char*>(a.kcache) + base), 0, n_bytes, kBufferWord3);
-  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char*>(reinterpret_cast<const char*>(a.vcache) + base), 0, n_bytes, kBufferWord3);
-#pragma unroll
-  for (int i = 0; i < T::KI; i++) {
-    const int j = wave + 8 * i;
-    if (i + 1 < T::KI || j < T::KW)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, FLK_LDS_PTR(k_buf + 256 * j), 16, t.k[i], 0, 0,
-                                               0);
-  }
-#pragma unroll
-  for (int i = 0; i < T::VI; i++)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, FLK_LDS_PTR(v_buf + 256 * (wave + 8 * i)), 16,
-                                             t.v[i], 0, 0, 0);
-}
-
-// The two LDS buffer pairs as four distinct LDS objects: the compiler then
-// sees that reads of one pair do not depend on loads in flight into the other.
-struct TileBuffers {
-  float* k0;
-  float* k1;
-  float* v0;
-  float* v1;
-};
-
-// s_waitcnt vmcnt(0), with expcnt and lgkmcnt left at their maxima.
-__device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 
 }  // namespace flk

@@ -164,7 +164,9 @@ int32_t flk_attn_decode(const float* q, const float* kcache, const float* vcache
  * kcache, vcache, o, Dims{n_heads, n_kv_heads, head_dim, n_queries, pos0}],
  * dispatch layer.ts:743-750). Query i (absolute position pos0 + i) attends
  * keys [0, pos0 + i]; the chunk's own rows must already be in the cache.
- * Tiled flash attention on fp32 MFMA, split over keys for long caches. */
+ * Tiled flash attention on the matrix cores in f32 precision (operands in
+ * three bf16 parts; fp32 MFMA for calls of little work), cut over keys where
+ * whole q tiles would leave the GPU idle. */
 int32_t flk_attn_prefill(const float* q, const float* kcache, const float* vcache, float* o,
                          uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
                          uint32_t n_queries, uint32_t pos0, void* ws, uint64_t ws_bytes);

@@ -395,6 +395,106 @@ def test_prefill_groups_5_6_7(rng, d, H, Hkv, nq, pos0):
     assert meets_bar(m), fmt(m)
 
 
+# (heads, kv heads, queries, pos0) of enough work for the split kernel, at the
+# edges of its 128-row q tiles, its 64-key tiles and the equal runs of key tiles
+# that workgroups take: whole and cut q tiles, runs that start and end inside
+# them, kv heads that 256 workgroups do not divide by, q tiles left partly
+# empty, MHA and MQA.
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("H,Hkv,nq,pos0", [
+    (16, 8, 1025, 0), (16, 8, 960, 64), (16, 8, 513, 448), (5, 5, 1537, 0), (5, 5, 513, 2500),
+    (8, 1, 1100, 130), (24, 3, 600, 511), (40, 40, 300, 0), (56, 8, 257, 1000),
+])
+def test_prefill_schedule_edges(rng, d, H, Hkv, nq, pos0):
+    nk = pos0 + nq
+    q = randn(rng, nq * H * d)
+    k, v = randn(rng, nk * Hkv * d), randn(rng, nk * Hkv * d)
+    got = _prefill(q, k, v, H, Hkv, d, nq, pos0)
+    want = oracle.attn_prefill(q, k, v, H, Hkv, d, nq, pos0)
+    m = metrics(got, want, cf.attention(q, k, v, H, Hkv, d, nq, pos0))
+    print(fmt(m))
+    # Against float64: sums of f32 products over up to ~1100 keys, rounding errors
+    # growing like their square root, within 64 roundings of the largest output
+    # (near-zero outputs make relative bounds depend on the draw).
+    assert m["gpu_abs_vs_f64"] < 64 * 2.0 ** -24 * np.abs(want).max(), fmt(m)
+
+
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("H,Hkv,nq", [(16, 8, 1600), (16, 16, 1530)])
+def test_prefill_of_many_q_tiles_runs_without_a_workspace(rng, d, H, Hkv, nq):
+    # The f32 kernel then takes the call; sums are rounded in another order: each
+    # is within 64 eps of the exact value.
+    q = dev(randn(rng, nq * H * d))
+    k, v = dev(randn(rng, nq * Hkv * d)), dev(randn(rng, nq * Hkv * d))
+    outs = []
+    for ws in (None, ops.Workspace(H, Hkv, d, nq, nq)):
+        o = empty(nq * H * d)
+        ops.attn_prefill(q, k, v, o, H, Hkv, d, nq, 0, ws)
+        outs.append(get(o, nq * H * d))
+    scale = np.abs(outs[1]).max()
+    assert np.max(np.abs(outs[0] - outs[1])) < 2 * 64 * 2.0 ** -24 * scale
+
+
+def _attention_f32(q, k, v, H, Hkv, d, nq, pos0):
+    """Causal attention in plain f32, as IEEE arithmetic has it for inputs that
+    are not finite."""
+    o = np.empty((nq, H, d), np.float32)
+    q, k, v = q.reshape(nq, H, d), k.reshape(-1, Hkv, d), v.reshape(-1, Hkv, d)
+    with np.errstate(all="ignore"):
+        for i in range(nq):
+            for h in range(H):
+                kv = h // (H // Hkv)
+                s = k[:pos0 + i + 1, kv] @ q[i, h] / np.float32(np.sqrt(d))
+                p = np.exp(s - s.max())
+                o[i, h] = p / p.sum() @ v[:pos0 + i + 1, kv]
+    return o.ravel()
+
+
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("nq,pos0", [(1025, 0), (200, 2000)])
+def test_prefill_inputs_that_are_not_finite(rng, d, nq, pos0):
+    # The three-part split of such an input is no number: the items that see
+    # one are computed in plain f32. kv head 0: a key whose score is -inf, which
+    # weighs nothing; 1: an infinite v; 2: a v above bf16's range; 3: a NaN key
+    # (its rows are NaN); 4: an infinite and a NaN v past some rows' last key; 5: a
+    # q row of +inf, with keys > 0 (inf - inf: NaN); 6, 7: untouched.
+    H, Hkv = 16, 8
+    nk = pos0 + nq
+    q = randn(rng, nq * H * d).reshape(nq, H, d)
+    k, v = (randn(rng, nk * Hkv * d).reshape(nk, Hkv, d) for _ in range(2))
+    q[:, :, 0] = np.abs(q[:, :, 0]) + 0.1
+    k[5, 0, 0] = -np.inf
+    v[7, 1, 3] = np.inf
+    v[9, 2, 4] = 3.4e38
+    k[pos0 + 11, 3, 2] = np.nan
+    v[pos0 + 13, 4, 1] = np.inf
+    v[pos0 + 14, 4, 2] = np.nan
+    q[8, 10] = np.inf
+    k[:, 5] = np.abs(k[:, 5])
+    q, k, v = q.ravel(), k.ravel(), v.ravel()
+    got = _prefill(q, k, v, H, Hkv, d, nq, pos0).reshape(nq, H, d)
+    want = _attention_f32(q, k, v, H, Hkv, d, nq, pos0).reshape(nq, H, d)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isinf(got), np.isinf(want))
+    finite = np.isfinite(want)
+    # f32 scores and weights of up to ~5 in magnitude, sums over nk keys.
+    err = np.abs(got[finite] - want[finite]) / np.maximum(1.0, np.abs(want[finite]))
+    assert err.max() < 1e-4
+
+
+@pytest.mark.parametrize("d", [128, 64])
+def test_prefill_of_tiny_values(rng, d):
+    # v around 2^-118: its later parts are below bf16's normal range, where the
+    # matrix cores read zeros. Outputs that small are computed in plain f32.
+    H, Hkv, nq = 16, 8, 1025
+    q = randn(rng, nq * H * d)
+    k, v = randn(rng, nq * Hkv * d), randn(rng, nq * Hkv * d)
+    s = np.float32(2.0 ** -118)
+    base = _prefill(q, k, v, H, Hkv, d, nq, 0)
+    got = _prefill(q, k, v * s, H, Hkv, d, nq, 0) / s
+    assert np.max(np.abs(got - base)) < 2e-6 * np.abs(base).max()
+
+
 def test_prefill_queries_match_decode(rng):
     # test_head.ts:321-351: prefill query `at` equals the decode reference over
     # keys 0..at -- proves the causal bound is pos0 + qi + 1.
