@@ -24,6 +24,12 @@ constexpr int kWave = 64;
 __device__ __forceinline__ float fma32(float a, float b, float c) {
   return (float)((double)a * (double)b + (double)c);
 }
+// s_barrier once this wave's LDS operations are done; unlike __syncthreads it
+// leaves loads from memory in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 __device__ __forceinline__ float rsqrt_once(float y) { return (float)(1.0 / sqrt((double)y)); }
 
 // ------------------------------------------------------------- lane shuffles --
@@ -367,6 +373,7 @@ struct Q8Fuse {
   float norm_eps = 0.f;
   const float* up = nullptr;         // x <- swiglu(x, up)
   const float* res = nullptr;        // o <- res + W x
+  float* normed = nullptr;           // the norm's output too (one token, q8_head_norm)
   float* act = nullptr;              // (gate, up) row pairs -> act = swiglu (<= 1024 columns)
 };
 hipError_t launch_q8_matvec(const uint8_t* qs, const uint16_t* scales, const float* x, float* o,
@@ -374,6 +381,8 @@ hipError_t launch_q8_matvec(const uint8_t* qs, const uint16_t* scales, const flo
                             float* best_val = nullptr, uint32_t* best_idx = nullptr,
                             uint32_t* n_workgroups = nullptr, const Q8Fuse* fuse = nullptr);
 uint32_t q8_max_workgroups(uint32_t n_rows, uint32_t n_cols);
+// Whether a head's projection forms the norm of x itself (Q8Fuse::normed).
+bool q8_head_norm(uint32_t n_rows, uint32_t n_cols);
 
 // op 0: swiglu(a, b); op 1: a + b (elementwise.wgsl).
 hipError_t launch_elementwise(int op, const float* a, const float* b, float* o, uint32_t n,

@@ -119,10 +119,4 @@ struct SplitTile {
   static constexpr int KP = kPlane / kPThreads;  // K slots (and V slots) a thread stages
 };
 
-// s_barrier once this wave's LDS operations are done; unlike __syncthreads it
-// leaves loads from memory in flight.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 }  // namespace flk

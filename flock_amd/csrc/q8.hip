@@ -103,6 +103,8 @@ struct Q8Args {
   // o, act[t][i] = swiglu(gate_i, up_i) (elementwise.wgsl:24-30). Needs two
   // or more rows per wave (at most 1024 columns).
   float* act;
+  // The fused norm's output is also written here (kernels of whole rows; null: not).
+  float* normed;
 };
 
 // swigluRef (ops_ref.ts:103-110): fr(fr(g / fr(1 + fr(exp(-g)))) * up).
@@ -291,13 +293,37 @@ __device__ __forceinline__ void q8_load_res(const Q8Args& a, uint32_t tok, uint3
   }
 }
 
+// The rmsnorm scale of a fused matvec; nv: the first batch of x, requested
+// before the weights. Each wave forms it by itself, except where a CU holds many
+// waves (tall matrices): there one wave of the workgroup does, since eight waves
+// per SIMD would spend 5 us of f64 work on it.
+template <bool PER_WG, class LOAD>
+__device__ __forceinline__ float q8_fused_scale(const Q8Args& a, const float (&nv)[kQ8NormBatch],
+                                                LOAD ld) {
+  __shared__ float s_scale;
+  auto scale = [&]() {
+    float p0 = 0.f, p1 = 0.f;
+    q8_rms_fold(nv, p0, p1);
+    return q8_rms_rest(p0, p1, a.n_cols, a.norm_eps, ld);
+  };
+  if (!PER_WG) return scale();
+  if (threadIdx.x < kWave) {
+    const float s = scale();
+    if (threadIdx.x == 0) s_scale = s;
+  }
+  lds_barrier();  // leaves the weights' loads in flight
+  return s_scale;
+}
+
 // P logical lanes per row, NB x blocks per lane in registers (NB * 64 >= the
 // row's block count). Grid: (workgroups over row groups, tokens).
 // FUSE: the input fusions (rmsnorm / swiglu) are compiled in.
 // LDS_TREE: the lane tree's exchanges through ds_bpermute (the LDS unit)
 // instead of DPP (the VALU): for very tall matrices (the LM head), where the
 // VALU is the busier unit and latency is hidden by many row groups.
-template <int P, int NB, bool FUSE, bool LDS_TREE = false>
+// HEAD (with FUSE): the norm's output is written to `normed` as well. (A flag of
+// the instance: the stores' branch would make the others wait for their loads.)
+template <int P, int NB, bool FUSE, bool LDS_TREE = false, bool HEAD = false>
 __global__ __launch_bounds__(kQ8Threads) void q8_matvec_kernel(Q8Args a) {
   constexpr int R = kWave / P;  // rows per wave per step
   constexpr int kQ8Unroll = q8_unroll<NB, FUSE>();
@@ -332,11 +358,7 @@ __global__ __launch_bounds__(kQ8Threads) void q8_matvec_kernel(Q8Args a) {
   // after the optional input fusion.
   float scale = 1.f;
   if (FUSE && FLK_Q8_NORM_FIRST) {
-    if (a.norm_gain != nullptr) {  // uniform
-      float p0 = 0.f, p1 = 0.f;
-      q8_rms_fold(nv, p0, p1);
-      scale = q8_rms_rest(p0, p1, a.n_cols, a.norm_eps, ldx);
-    }
+    if (a.norm_gain != nullptr) scale = q8_fused_scale<HEAD && LDS_TREE>(a, nv, ldx);  // uniform
   } else if (FUSE) {
     scale = q8_norm_scale(a, xt);
   }
@@ -361,6 +383,12 @@ __global__ __launch_bounds__(kQ8Threads) void q8_matvec_kernel(Q8Args a) {
       // Every load of the block first (float4s), then the arithmetic: a
       // per-element load-then-use sequence serialises 32 memory latencies.
       q8_fused_block(a, xt, tok_off, c0, scale, xr[j]);
+      if (HEAD && wave == 0 && sub == 0 && live[j]) {
+        float4* dst = reinterpret_cast<float4*>(a.normed + tok_off + c0);
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+          dst[i] = make_float4(xr[j][4 * i], xr[j][4 * i + 1], xr[j][4 * i + 2], xr[j][4 * i + 3]);
+      }
     }
   }
 
@@ -462,14 +490,14 @@ __device__ __forceinline__ float q8_half_pair(uint4 w, float scale, const float*
 #ifndef FLK_Q8_1K_UNROLL_FUSED
 #define FLK_Q8_1K_UNROLL_FUSED 2
 #endif
-template <bool FUSE>
+template <bool FUSE, bool LDS_TREE>
 constexpr int q8_unroll_1k() {
-  return FUSE ? FLK_Q8_1K_UNROLL_FUSED : FLK_Q8_1K_UNROLL;
+  return FUSE && !LDS_TREE ? FLK_Q8_1K_UNROLL_FUSED : FLK_Q8_1K_UNROLL;
 }
 
-template <bool FUSE, bool LDS_TREE>
+template <bool FUSE, bool LDS_TREE, bool HEAD = false>
 __global__ __launch_bounds__(kQ8Threads) void q8_matvec1k_kernel(Q8Args a) {
-  constexpr int UR = q8_unroll_1k<FUSE>();
+  constexpr int UR = q8_unroll_1k<FUSE, LDS_TREE>();
   constexpr uint32_t kNb = 32;  // blocks per row
   const int lane = threadIdx.x & 63;
   const int b = lane >> 1, h = lane & 1;
@@ -508,11 +536,7 @@ __global__ __launch_bounds__(kQ8Threads) void q8_matvec1k_kernel(Q8Args a) {
   // This lane's 16 inputs: columns 32 b + 16 h .. + 15, after the fusion.
   float scale = 1.f;
   if (FUSE && FLK_Q8_NORM_FIRST) {
-    if (a.norm_gain != nullptr) {  // uniform
-      float p0 = 0.f, p1 = 0.f;
-      q8_rms_fold(nv, p0, p1);
-      scale = q8_rms_rest(p0, p1, a.n_cols, a.norm_eps, ldx);
-    }
+    if (a.norm_gain != nullptr) scale = q8_fused_scale<HEAD && LDS_TREE>(a, nv, ldx);  // uniform
   } else if (FUSE) {
     scale = q8_norm_scale(a, xt);
   }
@@ -541,6 +565,12 @@ __global__ __launch_bounds__(kQ8Threads) void q8_matvec1k_kernel(Q8Args a) {
         }
         xr[4 * i + k] = v;
       }
+    }
+    if (HEAD && wave == 0) {
+      float4* dst = reinterpret_cast<float4*>(a.normed + tok_off + c0);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        dst[i] = make_float4(xr[4 * i], xr[4 * i + 1], xr[4 * i + 2], xr[4 * i + 3]);
     }
   }
 
@@ -1435,7 +1465,7 @@ static Q8MfmaPlan q8_mfma_plan(uint32_t n_rows, uint32_t n_cols, uint32_t n_toke
 // Workgroups: one resident wave of them (every CU filled to its occupancy
 // limit, so no workgroup waits for another to finish), never more than there
 // are row groups.
-template <int P, int NB, bool FUSE, bool LDS_TREE = false, bool K1 = false>
+template <int P, int NB, bool FUSE, bool LDS_TREE = false, bool K1 = false, bool HEAD = false>
 static uint32_t q8_grid_x(uint32_t n_groups) {
   static int per_cu = 0;
   if (per_cu == 0) {
@@ -1443,11 +1473,11 @@ static uint32_t q8_grid_x(uint32_t n_groups) {
     hipError_t e = hipSuccess;
     if (FLK_Q8_WG_PER_CU == 0) {
       if (K1)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, q8_matvec1k_kernel<FUSE, LDS_TREE>,
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, q8_matvec1k_kernel<FUSE, LDS_TREE, HEAD>,
                                                          kQ8Threads, 0);
       else
         e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &n, q8_matvec_kernel<P, NB, FUSE, LDS_TREE>, kQ8Threads, 0);
+            &n, q8_matvec_kernel<P, NB, FUSE, LDS_TREE, HEAD>, kQ8Threads, 0);
     }
     if (FLK_Q8_WG_PER_CU > 0 || e != hipSuccess || n < 1)
       n = FLK_Q8_WG_PER_CU > 0 ? FLK_Q8_WG_PER_CU : 2;
@@ -1462,7 +1492,7 @@ static uint32_t q8_grid_x(uint32_t n_groups) {
     cus = cus_of[dev];
   }
   const uint32_t per_wg =
-      (kQ8Threads / kWave) * (K1 ? q8_unroll_1k<FUSE>() : q8_unroll<NB, FUSE>());
+      (kQ8Threads / kWave) * (K1 ? q8_unroll_1k<FUSE, LDS_TREE>() : q8_unroll<NB, FUSE>());
   const uint32_t need = (n_groups + per_wg - 1) / per_wg;
   const uint32_t cap = (uint32_t)(per_cu * cus);
   return need < cap ? (need > 0 ? need : 1) : cap;
@@ -1471,6 +1501,12 @@ static uint32_t q8_grid_x(uint32_t n_groups) {
 template <int P, int NB>
 static uint32_t launch_q8(const Q8Args& a, hipStream_t st) {
   const uint32_t groups = (a.n_rows + (kWave / P) - 1) / (kWave / P);
+  if (a.normed != nullptr) {
+    const uint32_t gx = q8_grid_x<P, NB, true, false, false, true>(groups);
+    hipLaunchKernelGGL((q8_matvec_kernel<P, NB, true, false, true>), dim3(gx, a.n_tokens),
+                       dim3(kQ8Threads), 0, st, a);
+    return gx;
+  }
   if (a.norm_gain != nullptr || a.up != nullptr) {
     const uint32_t gx = q8_grid_x<P, NB, true>(groups);
     hipLaunchKernelGGL((q8_matvec_kernel<P, NB, true>), dim3(gx, a.n_tokens), dim3(kQ8Threads), 0,
@@ -1496,6 +1532,12 @@ static uint32_t launch_q8_1k(const Q8Args& a, hipStream_t st) {
     hipLaunchKernelGGL(kernel, dim3(gx, a.n_tokens), dim3(kQ8Threads), 0, st, a);
     return gx;
   };
+  if (a.normed != nullptr && a.n_rows >= kQ8LdsTreeRows)
+    return go(q8_matvec1k_kernel<true, true, true>,
+              q8_grid_x<32, 1, true, true, true, true>(groups));
+  if (a.normed != nullptr)
+    return go(q8_matvec1k_kernel<true, false, true>,
+              q8_grid_x<32, 1, true, false, true, true>(groups));
   if (a.norm_gain != nullptr || a.up != nullptr)
     return go(q8_matvec1k_kernel<true, false>, q8_grid_x<32, 1, true, false, true>(groups));
   if (a.n_rows >= kQ8LdsTreeRows)
@@ -1516,18 +1558,29 @@ uint32_t q8_max_workgroups(uint32_t n_rows, uint32_t n_cols) {
   return (groups + per_wg - 1) / per_wg;
 }
 
+// Tall matrices other than 1024 columns wide keep a launch for the norm: the
+// kernel that holds 32 columns per lane loses waves per SIMD to the norm's
+// registers (151936 x 2080, us, graph replay: 85 apart, 100 fused; 70000 x 256: 13.7,
+// 15.3; fused against apart where it is done: 151936 x 1024 33.3 / 36.3, 32000 x 2080
+// 26.7 / 30.2, 2000 x 1024 7.6 / 9.0).
+bool q8_head_norm(uint32_t n_rows, uint32_t n_cols) {
+  return n_cols / 32 <= (uint32_t)kQ8Lanes * kQ8MaxRegBlocks &&
+         (n_rows < kQ8LdsTreeRows || n_cols == 1024);
+}
+
 hipError_t launch_q8_matvec(const uint8_t* qs, const uint16_t* scales, const float* x, float* o,
                             uint32_t n_rows, uint32_t n_cols, uint32_t n_tokens,
                             hipStream_t st, float* best_val, uint32_t* best_idx,
                             uint32_t* n_workgroups, const Q8Fuse* fuse) {
   Q8Args a{qs, scales, x, o, n_rows, n_cols, n_tokens, best_val, best_idx,
-           nullptr, 0.f, nullptr, nullptr, nullptr};
+           nullptr, 0.f, nullptr, nullptr, nullptr, nullptr};
   if (fuse != nullptr) {
     a.norm_gain = fuse->norm_gain;
     a.norm_eps = fuse->norm_eps;
     a.up = fuse->up;
     a.res = fuse->res;
     a.act = fuse->act;
+    a.normed = fuse->normed;
   }
   const uint32_t nb = n_cols / 32;
   uint32_t gx;

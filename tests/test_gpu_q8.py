@@ -320,6 +320,38 @@ def test_lm_head_matches_oracle(rng, vocab, hidden):
     assert run_head(x, gain, packed, vocab, hidden, with_logits=False)[2:] == (w_v, w_i)
 
 
+@pytest.mark.parametrize("vocab,hidden", [
+    (500, 32), (333, 1024), (100, 2080), (40, 8192),  # short matrices, every row width
+    (65535, 64), (65536, 64), (65537, 1024),          # tall: apart, or one norm per workgroup
+    (40, 8224),                                       # too wide to hold x: its own norm launch
+])
+def test_lm_head_with_the_norm_fused_or_apart(rng, vocab, hidden):
+    """x and gain at 16-byte boundaries (the projection forms the norm) give the
+    bits of unaligned ones and of a norm in place (a launch of its own)."""
+    packed = random_packed(rng, vocab, hidden)
+    w = ops.Q8Matrix.from_packed(packed, vocab, hidden)
+    x = rng.standard_normal(hidden).astype(np.float32)
+    gain = rng.normal(1, 0.1, hidden).astype(np.float32)
+    ws = ops.DeviceBuffer(ops.lm_head_ws_bytes(vocab, hidden))
+
+    def run(x_off=0, gain_off=0, in_place=False):
+        xb, gb = (ops.DeviceBuffer.from_array(np.concatenate([np.zeros(o, np.float32), a]))
+                  for o, a in ((x_off, x), (gain_off, gain)))
+        normed = xb if in_place else ops.DeviceBuffer.from_array(np.full(hidden, np.nan, np.float32))
+        logits = ops.DeviceBuffer.from_array(np.full(vocab, np.nan, np.float32))
+        ov, oi = ops.DeviceBuffer(4), ops.DeviceBuffer(4)
+        ops.lm_head(xb.ptr + 4 * x_off, gb.ptr + 4 * gain_off, oracle.QWEN3_EPS, w, normed, logits,
+                    ov, oi, ws)
+        ops.sync()
+        return (normed.download(hidden), logits.download(vocab), ov.download(1),
+                oi.download(1, np.uint32))
+
+    want = run()
+    assert np.array_equal(want[0], oracle.rmsnorm(x, gain, hidden, 1, oracle.QWEN3_EPS))
+    for other in (run(x_off=1), run(gain_off=3), run(in_place=True)):
+        assert all(np.array_equal(a, b) for a, b in zip(want, other))
+
+
 def test_lm_head_tie_picks_lowest_row(rng):
     vocab, hidden = 151936, 1024
     packed = random_packed(rng, vocab, hidden).reshape(vocab, -1)
