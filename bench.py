@@ -380,6 +380,9 @@ class Prefill2k(Workload):
     unit = "TFLOP/s"
     bound = "mfma"
     kernel = "flk_attn_prefill: prefill_kernel<128> (equal runs of key tiles + prefill_merge_kernel)"
+    roofline_note = ("each f32 product is six bf16 MFMA ones, whose ceiling is 417 TFLOP/s: the "
+                     "fraction of the fp32 MFMA peak can pass 1; traffic was counted on the f32 "
+                     "kernel, before partials of cut q tiles")
 
     def __init__(self, torch, ops, n=2048, pos0=0, layers=1):
         self.torch, self.ops = torch, ops
@@ -801,9 +804,8 @@ def random_q8(rng, rows, cols, scale=8e-4):
 class Q8Prefill(Workload):
     """The largest projection of a 2048-token prefill: ffn_norm, then gate and
     up (3072 x 1024 each, rows interleaved) with SwiGLU, in one
-    flk_q8_gate_up_swiglu call over 2048 tokens -- the weight-reusing tile
-    kernel (q8_mm_kernel), exact to the coop(64) order. VALU-bound: the
-    exact summation order rules out MFMA."""
+    flk_q8_gate_up_swiglu call over 2048 tokens -- q8_mfma_kernel, exact to the
+    coop(64) order: f32 MFMAs form its dot4s, the VALU does the rest of it."""
 
     data = ("synthetic: random Q8_0 weights of the Qwen3-0.6B shapes (seeded quants, f16 "
             "scales), seeded N(0,1) inputs, zeroed or seeded caches")
@@ -811,8 +813,7 @@ class Q8Prefill(Workload):
     name = "q8prefill"
     unit = "TFLOP/s"
     bound = "valu"
-    kernel = ("flk_q8_gate_up_swiglu: q8_mm1_kernel<kMmNorm> (32 rows x 8 tokens per tile, "
-              "8 row tiles per workgroup)")
+    kernel = "flk_q8_gate_up_swiglu: q8_mfma_kernel<4, kMmNorm> (64 rows x 64 tokens per tile)"
     n_tokens, ffn, hid = 2048, 3072, 1024
 
     def __init__(self, torch, ops):
