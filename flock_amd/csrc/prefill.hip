@@ -59,13 +59,33 @@
 
 namespace flk {
 
+// ---- inputs that three bf16 parts do not cover -----------------------------------
+// A row of an item is formed again in plain f32 (row_f32) where the parts lose
+// something; what decides is the row's own result:
+// - an output that is no finite number: an infinity or NaN in q, K or V, or a
+//   magnitude that bf16 rounds to infinity, splits into infinite - infinite. What
+//   f32 arithmetic makes of such inputs (a -inf score weighs nothing, an infinite v
+//   gives an infinite output) is formed here.
+// - v whose later parts fall below bf16's range: an output other than 0 below
+//   kTinyOutput.
+// A v that is not finite past a row's last key reaches the row too (0 x infinite):
+// its result is the one of its own keys, but its last bits may differ.
+constexpr float kTinyOutput = 0x1p-100f;
+
+// What a workgroup's waves tell each other about such rows, in LDS.
+struct Redo {
+  uint32_t any;              // some row is to be formed again
+  uint32_t bad[kRows / 32];  // which
+  uint32_t no_nan_key;       // ~(the first key of the item with a NaN in K)
+};
+
 // One row's attention over keys key0 .. key1 - 1 in plain f32 by one wave: lane
 // = key for the scores, lane = channels for the sums. Returns (m, l) and, in
 // lane l, channels l, l + 64, ... of the unnormalised sum.
 template <int D>
-__device__ void row_f32(const PrefillArgs& a, const float* qrow, uint32_t kvh, uint32_t key0,
-                        uint32_t key1, float& m, float& l, float (&acc)[D / 64]) {
-  const uint32_t lane = threadIdx.x & 63;
+__device__ void row_f32(const PrefillArgs& a, uint32_t lane, const float* qrow, uint32_t kvh,
+                        uint32_t key0, uint32_t key1, float& m, float& l,
+                        float (&acc)[D / 64]) {
   const size_t stride = (size_t)a.n_kv_heads * D;
   const float* kb = a.kcache + (size_t)kvh * D;
   const float* vb = a.vcache + (size_t)kvh * D;
@@ -77,9 +97,17 @@ __device__ void row_f32(const PrefillArgs& a, const float* qrow, uint32_t kvh, u
     const uint32_t key = k0 + lane;
     float s = -INFINITY;
     if (key < key1) {
+      const float4* kr = reinterpret_cast<const float4*>(kb + key * stride);
+      const float4* qr = reinterpret_cast<const float4*>(qrow);
       s = 0.f;
-      for (int c = 0; c < D; c++)
-        s = fmaf(kb[key * stride + c], qrow[c] * a.scale_log2e, s);
+#pragma unroll 4
+      for (int c = 0; c < D / 4; c++) {
+        const float4 k = kr[c], q = qr[c];
+        s = fmaf(k.x, q.x * a.scale_log2e, s);
+        s = fmaf(k.y, q.y * a.scale_log2e, s);
+        s = fmaf(k.z, q.z * a.scale_log2e, s);
+        s = fmaf(k.w, q.w * a.scale_log2e, s);
+      }
     }
     float mx = s;
 #pragma unroll
@@ -96,46 +124,76 @@ __device__ void row_f32(const PrefillArgs& a, const float* qrow, uint32_t kvh, u
 #pragma unroll
     for (int x = 32; x >= 1; x >>= 1) sum += shfl_xor(sum, x);
     l += sum;
+    float blk[D / 64];  // of these keys: a long sum is rounded once per 64 keys
+#pragma unroll
+    for (int c = 0; c < D / 64; c++) blk[c] = 0.f;
     const uint32_t n = min(key1 - k0, 64u);
+#pragma unroll 8
     for (uint32_t j = 0; j < n; j++) {
-      const float pj = __shfl(p, j, kWave);
+      const float pj = __builtin_bit_cast(
+          float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), j));
 #pragma unroll
       for (int c = 0; c < D / 64; c++)
-        acc[c] = fmaf(pj, vb[(k0 + j) * stride + 64 * c + lane], acc[c]);
+        blk[c] = fmaf(pj, vb[(k0 + j) * stride + 64 * c + lane], blk[c]);
     }
+#pragma unroll
+    for (int c = 0; c < D / 64; c++) acc[c] += blk[c];
+    if (l != l) return;  // NaN in every channel, whatever follows
   }
 }
 
-// An item again in plain f32, for the inputs that three bf16 parts do not
-// cover. Slow, and only then:
-// - no number (an infinity or NaN in q, K or V, or a magnitude that bf16 rounds
-//   to infinity): infinite - infinite shows up as a NaN in the item's output,
-//   and what f32 arithmetic makes of such inputs (a -inf score has weight 0, an
-//   infinite v gives an infinite output) is formed here;
-// - v whose later parts fall below 2^-126, which the matrix cores read as 0: an
-//   output of less than kTinyOutput in magnitude. (Above it that costs less
-//   than 2^-24 of the output; in scores it is lost against 1.)
-constexpr float kTinyOutput = 0x1p-100f;
+// Where redo_rows puts row r's channels and (m, l): in two tiles of the ring.
 template <int D>
-__device__ void item_f32(const PrefillArgs a, uint32_t kvh, uint32_t qt,
-                                      uint32_t kt0, uint32_t kt1, bool final, size_t slot) {
-  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (uint32_t r = wave; r < a.q_per_tile * a.group; r += kPThreads / 64) {
-    const uint32_t qi = qt * a.q_per_tile + r / a.group;
-    const uint32_t h = kvh * a.group + r % a.group;
-    if (qi >= a.n_queries) break;
-    const size_t row = ((size_t)qi * a.n_heads + h) * D;
-    float m, l, acc[D / 64];
-    row_f32<D>(a, a.q + row, kvh, kt0 * kBK, min(kt1 * kBK, a.pos0 + qi + 1), m, l, acc);
-#pragma unroll
-    for (int c = 0; c < D / 64; c++) {
-      if (final)
-        a.o[row + 64 * c + lane] = acc[c] / l;
-      else
-        a.part_acc[(slot * kRows + r) * D + 64 * c + lane] = acc[c];
-    }
-    if (!final && lane == 0) a.part_ml[slot * kRows + r] = make_float2(m, l);
+__device__ __forceinline__ float* row_lds(uint32x4* const (&buf)[2], uint32_t r) {
+  return reinterpret_cast<float*>(buf[r / (kRows / 2)]) + r % (kRows / 2) * D;
+}
+template <int D>
+__device__ __forceinline__ float2* ml_lds(uint32x4* const (&buf)[2]) {
+  static_assert(kRows / 2 * D / 4 + kRows / 2 <= SplitTile<D>::kSlots, "rows and (m, l) fit");
+  return reinterpret_cast<float2*>(buf[1] + kRows / 2 * D / 4);
+}
+
+// Forms the rows of `s` again, into LDS: channels (divided by l when `final`) and
+// (m, l). Rows that see a NaN in K are NaN already and leave s, so that a NaN token
+// costs little; other rows cost a wave the reads of all their keys, 20 us per 64
+// keys with every CU at it. 16 / 8 heads of 128, us, 2048 and 8192 tokens: 117, 1297;
+// a NaN token half way 138, 1500; an infinite v that every row sees 3480, 82000 (on
+// the f32 kernel, which it does not slow: 157, 2100).
+template <int D>
+__device__ void redo_rows(const PrefillArgs& a, Redo& s, uint32x4* const (&buf)[2], uint32_t kvh,
+                          uint32_t qt, uint32_t kt0, uint32_t kt1, bool final) {
+  uint32_t tid = threadIdx.x;  // opaque: nothing of this is formed for every item
+  asm volatile("" : "+v"(tid));
+  const uint32_t lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t key0 = kt0 * kBK, key1 = min(kt1 * kBK, a.pos0 + a.n_queries);
+  constexpr int CH = D / 4;
+  uint32_t nan_key = ~0u;
+#pragma unroll 4
+  for (uint32_t key = key0 + tid / CH; key < key1; key += kPThreads / CH) {
+    const float4 k = *reinterpret_cast<const float4*>(
+        a.kcache + ((size_t)key * a.n_kv_heads + kvh) * D + 4 * (tid % CH));
+    if (k.x != k.x || k.y != k.y || k.z != k.z || k.w != k.w) nan_key = min(nan_key, key);
   }
+  if (nan_key != ~0u) atomicMax(&s.no_nan_key, ~nan_key);
+  __syncthreads();
+  nan_key = ~s.no_nan_key;
+  for (uint32_t r = wave; r < a.q_per_tile * a.group; r += kPThreads / 64) {
+    const uint32_t bit = 1u << r % 32, pos = a.pos0 + qt * a.q_per_tile + r / a.group;
+    if (!(s.bad[r / 32] & bit)) continue;
+    if (pos >= nan_key) {
+      if (lane == 0) atomicAnd(&s.bad[r / 32], ~bit);
+      continue;
+    }
+    const float* q = a.q + ((size_t)(pos - a.pos0) * a.n_heads + kvh * a.group + r % a.group) * D;
+    float m, l, acc[D / 64];
+    row_f32<D>(a, lane, q, kvh, key0, min(key1, pos + 1), m, l, acc);
+#pragma unroll
+    for (int i = 0; i < D / 64; i++)
+      row_lds<D>(buf, r)[64 * i + lane] = final ? acc[i] / l : acc[i];
+    if (lane == 0) ml_lds<D>(buf)[r] = make_float2(m, l);
+  }
+  __syncthreads();
 }
 
 // Key tiles on their way to LDS: this thread's share of one K and one V tile.
@@ -283,7 +341,7 @@ struct Pipe {
 // nxt_qt's rows are requested under the combine; without a next item the caller
 // names a tile of this one.
 template <int D>
-__device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, int* s_bad, uint32_t kvh,
+__device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo* redo, uint32_t kvh,
                                          uint32_t qt, uint32_t kt0, uint32_t kt1, bool final,
                                          size_t slot, const TileLoader<D>& ld, uint32_t nxt_qt,
                                          uint32_t nxt_kt) {
@@ -403,7 +461,8 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, int* 
     if (__builtin_amdgcn_ballot_w64(lmx > m_run + 8.f) != 0) {  // uniform branch
       // Only rows whose own maximum passed the threshold move their reference;
       // the others keep it and are multiplied by exactly 1, so a row's result
-      // depends on its own keys only (causality holds bit for bit).
+      // depends on its own keys only (causality holds bit for bit, but for a v
+      // that is not finite past the row's last key: row_f32).
       const float mx = max_xor<32>(lmx);
       const bool up = mx > m_run + 8.f;
       const float corr = up ? __builtin_amdgcn_exp2f(m_run - mx) : 1.f;
@@ -479,7 +538,8 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, int* 
           uint32x4, make_float4(give[4 * j], give[4 * j + 1], give[4 * j + 2], give[4 * j + 3]));
   }
   if (lg == 0) ml_x[half * kRows + r] = make_float2(m_run, l_run);
-  if (threadIdx.x == 0) *s_bad = 0;
+  if (threadIdx.x < sizeof(Redo) / 4)
+    reinterpret_cast<uint32_t*>(redo)[threadIdx.x] = 0;
   lds_barrier();
   const float2 ml2 = ml_x[(1 - half) * kRows + r];
   const float M = fmaxf(m_run, ml2.x);
@@ -489,44 +549,87 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, int* 
   const float w1 = __builtin_amdgcn_exp2f(m_run - M);
   const float w2 = __builtin_amdgcn_exp2f(ml2.x - M);
   const float L = l_run * w1 + ml2.y * w2;
-  float* dst;
-  if (final) {
-    dst = a.o + row.offset(a);
-  } else {
-    dst = a.part_acc + (slot * kRows + r) * D;
-    if (lg == 0 && half == 0) a.part_ml[slot * kRows + r] = make_float2(M, L);
-  }
-  bool bad = false;
-  auto redo = [](float x) { return !(fabsf(x) >= kTinyOutput) && x != 0.f; };
 #pragma unroll
   for (int c = 0; c < HB; c++)
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       const float4 x = __builtin_bit_cast(
           float4, (half ? bv : bn)[(((wave & 3) * HB + c) * 4 + j) * 64 + lane]);
-      float4 v = make_float4(mine[c][4 * j] * w1 + x.x * w2, mine[c][4 * j + 1] * w1 + x.y * w2,
-                             mine[c][4 * j + 2] * w1 + x.z * w2,
-                             mine[c][4 * j + 3] * w1 + x.w * w2);
-      if (final) v = make_float4(v.x / L, v.y / L, v.z / L, v.w / L);
-      bad |= redo(v.x) || redo(v.y) || redo(v.z) || redo(v.w);
-      if (row_ok || !final)
-        *reinterpret_cast<float4*>(dst + 32 * (HB * half + c) + 8 * j + 4 * lg) = v;
+      mine[c][4 * j] = mine[c][4 * j] * w1 + x.x * w2;
+      mine[c][4 * j + 1] = mine[c][4 * j + 1] * w1 + x.y * w2;
+      mine[c][4 * j + 2] = mine[c][4 * j + 2] * w1 + x.z * w2;
+      mine[c][4 * j + 3] = mine[c][4 * j + 3] * w1 + x.w * w2;
     }
-  bad |= !final && L != L;
-  if (row_ok && bad) *s_bad = 1;
-  // Every wave is done with the exchange (the next item's V goes there), and its
-  // stores are out before item_f32's.
-  __syncthreads();
-  if (*s_bad) {
-    item_f32<D>(a, kvh, qt, kt0, kt1, final, slot);
-    __syncthreads();
+  if (final) {  // uniform
+#pragma unroll
+    for (int c = 0; c < HB; c++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) mine[c][i] = mine[c][i] / L;
+  }
+  float least = INFINITY, most = 0.f;  // magnitudes; a NaN stays in `most`
+#pragma unroll
+  for (int c = 0; c < HB; c++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      least = fminf(least, fabsf(mine[c][i]));
+      most = __builtin_elementwise_maximum(most, fabsf(mine[c][i]));
+    }
+  bool again = row_ok && (!(most < INFINITY) || !(least >= kTinyOutput || least == 0.f));
+  if (__builtin_amdgcn_ballot_w64(again) != 0) {  // uniform
+    least = INFINITY;  // of the others than 0
+#pragma unroll
+    for (int c = 0; c < HB; c++)
+#pragma unroll
+      for (int i = 0; i < 16; i++)
+        least = fminf(least, mine[c][i] != 0.f ? fabsf(mine[c][i]) : INFINITY);
+    again = row_ok && (!(most < INFINITY) || least < kTinyOutput);
+    if (again) {
+      atomicOr(&redo->bad[wave & 3], 1u << lc);
+      redo->any = 1;
+    }
+  }
+  auto store = [&](float2 ml) {
+    float* dst;
+    if (final) {
+      dst = a.o + row.offset(a);
+    } else {
+      dst = a.part_acc + (slot * kRows + r) * D;
+      if (lg == 0 && half == 0) a.part_ml[slot * kRows + r] = ml;
+    }
+#pragma unroll
+    for (int c = 0; c < HB; c++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        *reinterpret_cast<float4*>(dst + 32 * (HB * half + c) + 8 * j + 4 * lg) =
+            make_float4(mine[c][4 * j], mine[c][4 * j + 1], mine[c][4 * j + 2],
+                        mine[c][4 * j + 3]);
+  };
+  if (!again && (row_ok || !final)) store(make_float2(M, L));
+  __syncthreads();  // every wave is done with the exchange (the next item's V goes there)
+  if (redo->any) {  // uniform
+    uint32x4* const buf[2] = {bv, bn};
+    redo_rows<D>(a, *redo, buf, kvh, qt, kt0, kt1, final);
+    float2 ml = make_float2(M, L);
+    if (redo->bad[wave & 3] >> lc & 1) {  // also where this lane's channels are stored
+      again = true;
+      const float* x = row_lds<D>(buf, r) + 32 * HB * half + 4 * lg;
+#pragma unroll
+      for (int c = 0; c < HB; c++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) mine[c][i] = x[32 * c + 8 * (i / 4) + i % 4];
+      ml = ml_lds<D>(buf)[r];
+    }
+    if (again) store(ml);
+    // Requested again, so that nothing else is held over redo_rows.
+    QRow<D>(a, kvh, nxt_qt).fetch(p.q, a);
+    ld.load_v(st, a, kvh, nxt_kt);
   }
 }
 
 template <int D>
 __global__ __launch_bounds__(kPThreads, 2) void prefill_kernel(PrefillArgs a, PrefillTable tab) {
   __shared__ uint32x4 lds[3 * SplitTile<D>::kSlots];
-  __shared__ int s_bad;
+  __shared__ Redo redo;
   const uint32_t kvh = blockIdx.x % a.n_kv_heads;
   const uint32_t w = blockIdx.x / a.n_kv_heads;
   const TileLoader<D> ld(a.n_kv_heads * D * 4);
@@ -551,7 +654,7 @@ __global__ __launch_bounds__(kPThreads, 2) void prefill_kernel(PrefillArgs a, Pr
     // A workgroup's first piece of a cut q tile has slot 2w, its last 2w + 1.
     const size_t slot = (size_t)(2 * w + (seq != s0.seq ? 1 : 0)) * a.n_kv_heads + kvh;
     const bool more = live(seq + 1, 0);
-    run_item<D>(a, p, &s_bad, kvh, qt, kt0, kt1, kt0 == 0 && kt1 == n_kt, slot, ld,
+    run_item<D>(a, p, &redo, kvh, qt, kt0, kt1, kt0 == 0 && kt1 == n_kt, slot, ld,
                 more ? prefill_seq_qt(seq + 1, a.n_qtiles) : qt, more ? 0 : kt0);
     seq++;
     kt0 = 0;

@@ -495,6 +495,27 @@ def test_prefill_of_tiny_values(rng, d):
     assert np.max(np.abs(got - base)) < 2e-6 * np.abs(base).max()
 
 
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("nq,pos0", [(1025, 0), (200, 2000)])
+def test_prefill_rows_keep_their_bits_beside_others_that_are_not_finite(rng, d, nq, pos0):
+    # Query 300 (or 30) is NaN, a key of a later position NaN, a query infinite:
+    # rows that do not see them have the bits that they have without them.
+    H, Hkv = 16, 8
+    nk, at = pos0 + nq, 30 if pos0 else 300
+    q = randn(rng, nq * H * d).reshape(nq, H, d)
+    k, v = (randn(rng, nk * Hkv * d).reshape(nk, Hkv, d) for _ in range(2))
+    base = _prefill(q.ravel(), k.ravel(), v.ravel(), H, Hkv, d, nq, pos0).reshape(nq, H, d)
+    q[at, 0, 5] = np.nan
+    q[at + 1, 2, 7] = np.inf
+    k[pos0 + at, 4, 3] = np.nan
+    got = _prefill(q.ravel(), k.ravel(), v.ravel(), H, Hkv, d, nq, pos0).reshape(nq, H, d)
+    same = np.ones((nq, H), bool)
+    same[at, 0] = same[at + 1, 2] = False
+    same[at:, 8:10] = False  # heads 8, 9 read kv head 4
+    assert np.array_equal(got[same], base[same])
+    assert np.all(np.isnan(got[at, 0])) and np.all(np.isnan(got[at:, 8:10]))
+
+
 def test_prefill_queries_match_decode(rng):
     # test_head.ts:321-351: prefill query `at` equals the decode reference over
     # keys 0..at -- proves the causal bound is pos0 + qi + 1.
