@@ -66,11 +66,15 @@ namespace flk {
 //   magnitude that bf16 rounds to infinity, splits into infinite - infinite. What
 //   f32 arithmetic makes of such inputs (a -inf score weighs nothing, an infinite v
 //   gives an infinite output) is formed here.
-// - v whose later parts fall below bf16's range: an output other than 0 below
-//   kTinyOutput.
+// - a normalised output other than 0 below kTinyOutput: parts end at 2^-133, bf16's
+//   smallest number (the matrix cores keep it), so lost parts of v cost an output up
+//   to 2^-134, i.e. up to 2^-26 of itself above that. (A v below 2^-134 counts as 0
+//   where no output of the row shows it.)
+// Weights lose as little: one below 2^-110 of the row's largest is off by up to 2^-134
+// of that (and one below 2^-126 is 0, as in the f32 kernel).
 // A v that is not finite past a row's last key reaches the row too (0 x infinite):
 // its result is the one of its own keys, but its last bits may differ.
-constexpr float kTinyOutput = 0x1p-100f;
+constexpr float kTinyOutput = 0x1p-108f;
 
 // What a workgroup's waves tell each other about such rows, in LDS.
 struct Redo {
@@ -574,7 +578,8 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo*
       least = fminf(least, fabsf(mine[c][i]));
       most = __builtin_elementwise_maximum(most, fabsf(mine[c][i]));
     }
-  bool again = row_ok && (!(most < INFINITY) || !(least >= kTinyOutput || least == 0.f));
+  const float tiny = final ? kTinyOutput : kTinyOutput * L;
+  bool again = row_ok && (!(most < INFINITY) || !(least >= tiny));
   if (__builtin_amdgcn_ballot_w64(again) != 0) {  // uniform
     least = INFINITY;  // of the others than 0
 #pragma unroll
@@ -582,7 +587,7 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo*
 #pragma unroll
       for (int i = 0; i < 16; i++)
         least = fminf(least, mine[c][i] != 0.f ? fabsf(mine[c][i]) : INFINITY);
-    again = row_ok && (!(most < INFINITY) || least < kTinyOutput);
+    again = row_ok && (!(most < INFINITY) || least < tiny);
     if (again) {
       atomicOr(&redo->bad[wave & 3], 1u << lc);
       redo->any = 1;

@@ -516,6 +516,75 @@ def test_prefill_rows_keep_their_bits_beside_others_that_are_not_finite(rng, d, 
     assert np.all(np.isnan(got[at, 0])) and np.all(np.isnan(got[at:, 8:10]))
 
 
+# (heads, kv heads, queries, pos0): cut q tiles, and whole ones.
+EXTREMES = [(16, 8, 1025, 0), (280, 40, 270, 0)]
+
+
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("H,Hkv,nq,pos0", EXTREMES)
+@pytest.mark.parametrize("bits", [100, 110, 118])
+def test_prefill_weights_far_below_the_largest(rng, d, H, Hkv, nq, pos0, bits):
+    # Key 0 takes nearly all the weight but its v is 0: outputs are what the
+    # others, `bits` powers of two below, make of large v. A score carries an f32's
+    # rounding, 2^-24 of it, into the exponent (at most 1e-5 here), sums are within 64
+    # eps, and a weight's parts end at 2^-133: half of that is lost.
+    q = np.zeros((nq, H, d), np.float32)
+    k, v = np.zeros((nq, Hkv, d), np.float32), np.empty((nq, Hkv, d), np.float32)
+    q[..., 0] = (bits + 0.3) * np.sqrt(d) * np.log(2)
+    k[0, :, 0] = 1
+    v[...] = (1 + rng.random((nq, Hkv, d))) * 2.0 ** 30
+    v[0] = 0
+    got = _prefill(q.ravel(), k.ravel(), v.ravel(), H, Hkv, d, nq, pos0).astype(np.float64)
+    want = cf.attention(q.ravel(), k.ravel(), v.ravel(), H, Hkv, d, nq, pos0)
+    tol = 1.4e-5 + 2.0 ** (bits + 0.3 - 134)
+    assert np.max(np.abs(got - want) / np.maximum(want, 2.0 ** -100)) < tol
+
+
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("H,Hkv,nq,pos0", EXTREMES + [(16, 8, 200, 4000)])
+@pytest.mark.parametrize("e", [-112, -109, -104, -99, 100])
+def test_prefill_of_equal_values_of_extreme_magnitude(rng, d, H, Hkv, nq, pos0, e):
+    # Every key alike, so that a sum of weights is the number of keys, and every
+    # v of a channel the same x 2^e: x is returned, to the rounding of such a
+    # sum (as in test_prefill_of_tiny_values). The x have large third parts.
+    nk = pos0 + nq
+    q = randn(rng, nq * H * d)
+    k = np.broadcast_to(randn(rng, Hkv * d), (nk, Hkv * d)).ravel()
+    x = (np.float32(1 + 2.0 ** -9 + 2.0 ** -17 - 2.0 ** -23)
+         * rng.choice(np.float32([-1, 1]), (1, Hkv, d))).astype(np.float32)
+    v = np.broadcast_to(x, (nk, Hkv, d)).ravel()
+    s = np.float32(2.0 ** e)
+    base = _prefill(q, k, v, H, Hkv, d, nq, pos0)
+    got = _prefill(q, k, v * s, H, Hkv, d, nq, pos0) / s
+    assert np.max(np.abs(got - base)) < 2e-6
+
+
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("H,Hkv,nq,pos0", EXTREMES)
+@pytest.mark.parametrize("which", ["all", "one channel", "late"])
+def test_prefill_of_subnormal_values(rng, d, H, Hkv, nq, pos0, which):
+    # v around 2^-130, below f32's normal range: outputs within the rounding of
+    # every product and of every sum to a multiple of 2^-149, and within the 2^-134
+    # below which a v alone in its row counts as 0.
+    q, k = randn(rng, nq * H * d), randn(rng, nq * Hkv * d)
+    v = randn(rng, nq * Hkv * d).reshape(nq, Hkv, d)
+    base = _prefill(q, k, v.ravel(), H, Hkv, d, nq, pos0).reshape(nq, H, d)
+    c = slice(None) if which == "all" else slice(7, 8)
+    r = slice(nq // 2, None) if which == "late" else slice(None)
+    v1 = v.copy()
+    v1[..., c] = 0
+    v1[r, :, c] = v[r, :, c] * np.float32(2.0 ** -130)
+    got = _prefill(q, k, v1.ravel(), H, Hkv, d, nq, pos0).reshape(nq, H, d)
+    want = cf.attention(q, k, v1.ravel(), H, Hkv, d, nq, pos0).reshape(nq, H, d)
+    assert np.max(np.abs(got[..., c] - want[..., c])) < 40 * 2.0 ** -149 + 2.0 ** -134
+    if which != "all":  # the other channels
+        rest = np.arange(d) != 7
+        assert np.max(np.abs(got[..., rest] - base[..., rest])) < 2e-6 * np.abs(base).max()
+    if which == "late":  # rows that see none of it, and their zeros
+        assert np.array_equal(got[:nq // 2][..., rest], base[:nq // 2][..., rest])
+        assert not got[:nq // 2, :, 7].any()
+
+
 def test_prefill_queries_match_decode(rng):
     # test_head.ts:321-351: prefill query `at` equals the decode reference over
     # keys 0..at -- proves the causal bound is pos0 + qi + 1.
