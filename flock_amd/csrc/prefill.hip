@@ -61,20 +61,23 @@ namespace flk {
 
 // ---- inputs that three bf16 parts do not cover -----------------------------------
 // A row of an item is formed again in plain f32 (row_f32) where the parts lose
-// something; what decides is the row's own result:
+// something; what decides is the row's own q and its own result:
 // - an output that is no finite number: an infinity or NaN in q, K or V, or a
 //   magnitude that bf16 rounds to infinity, splits into infinite - infinite. What
 //   f32 arithmetic makes of such inputs (a -inf score weighs nothing, an infinite v
 //   gives an infinite output) is formed here.
-// - a normalised output other than 0 below kTinyOutput: parts end at 2^-133, bf16's
-//   smallest number (the matrix cores keep it), so lost parts of v cost an output up
-//   to 2^-134, i.e. up to 2^-26 of itself above that. (A v below 2^-134 counts as 0
+// - q with an element other than 0 below kTinyQ, or one of at least kLargeQ. Parts end
+//   at 2^-133, bf16's smallest number (the matrix cores keep it), so a value of less
+//   than 2^-110 loses up to 2^-134, which costs a score that times the other factor:
+//   with no part of q lost, at most D 2^-134 kLargeQ = 2^-27.
+// - a normalised output other than 0 below kTinyOutput: lost parts of v cost it up to
+//   2^-134, i.e. up to 2^-26 of itself above that. (A v below 2^-134 counts as 0
 //   where no output of the row shows it.)
 // Weights lose as little: one below 2^-110 of the row's largest is off by up to 2^-134
 // of that (and one below 2^-126 is 0, as in the f32 kernel).
 // A v that is not finite past a row's last key reaches the row too (0 x infinite):
 // its result is the one of its own keys, but its last bits may differ.
-constexpr float kTinyOutput = 0x1p-108f;
+constexpr float kTinyOutput = 0x1p-108f, kTinyQ = 0x1p-110f, kLargeQ = 0x1p100f;
 
 // What a workgroup's waves tell each other about such rows, in LDS.
 struct Redo {
@@ -369,6 +372,7 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo*
   // The row's q, pre-multiplied by scale * log2(e) so that S^T comes out in
   // base-2 units, split.
   uint32x4 qf[NG][3];
+  uint32_t q_mid = ~0u;  // bits 14 and 30: every element's top two exponent bits differ
 #pragma unroll
   for (int j = 0; j < NG; j++) {
     const float4 x = p.q[2 * j], y = p.q[2 * j + 1];
@@ -379,7 +383,27 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo*
       split_pair(e[2 * i] * a.scale_log2e, e[2 * i + 1] * a.scale_log2e, u);
 #pragma unroll
       for (int k = 0; k < 3; k++) qf[j][k][i] = u[k];
+      q_mid &= u[0] ^ (u[0] << 1);
     }
+  }
+  // 2^-63 <= |q| < 2^65 has top exponent bits 01 or 10; a row with others (or
+  // zeros) is read again and looked at.
+  bool q_out = false;
+  if (__builtin_amdgcn_ballot_w64((q_mid & 0x40004000u) != 0x40004000u) != 0) {  // uniform
+    float4 q[D / 8];
+    row.fetch(q, a);
+    float least = 1.f, most = 0.f;  // magnitudes other than 0; a NaN stays in `most`
+#pragma unroll
+    for (int j = 0; j < D / 8; j++) {
+      const float e[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float x = fabsf(e[i] * a.scale_log2e);
+        least = fminf(least, x != 0.f ? x : 1.f);
+        most = __builtin_elementwise_maximum(most, x);
+      }
+    }
+    q_out = least < kTinyQ || !(most < kLargeQ);
   }
   lds_barrier();
 
@@ -579,7 +603,7 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo*
       most = __builtin_elementwise_maximum(most, fabsf(mine[c][i]));
     }
   const float tiny = final ? kTinyOutput : kTinyOutput * L;
-  bool again = row_ok && (!(most < INFINITY) || !(least >= tiny));
+  bool again = row_ok && (q_out || !(most < INFINITY) || !(least >= tiny));
   if (__builtin_amdgcn_ballot_w64(again) != 0) {  // uniform
     least = INFINITY;  // of the others than 0
 #pragma unroll
@@ -587,7 +611,7 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo*
 #pragma unroll
       for (int i = 0; i < 16; i++)
         least = fminf(least, mine[c][i] != 0.f ? fabsf(mine[c][i]) : INFINITY);
-    again = row_ok && (!(most < INFINITY) || least < tiny);
+    again = row_ok && (q_out || !(most < INFINITY) || least < tiny);
     if (again) {
       atomicOr(&redo->bad[wave & 3], 1u << lc);
       redo->any = 1;

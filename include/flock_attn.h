@@ -166,7 +166,11 @@ int32_t flk_attn_decode(const float* q, const float* kcache, const float* vcache
  * keys [0, pos0 + i]; the chunk's own rows must already be in the cache.
  * Tiled flash attention on the matrix cores in f32 precision (operands in
  * three bf16 parts; fp32 MFMA for calls of little work), cut over keys where
- * whole q tiles would leave the GPU idle. */
+ * whole q tiles would leave the GPU idle. Range: rows whose q or output holds
+ * an infinity, a NaN or extreme magnitudes (q from 2^100 or below 2^-110, an
+ * output below 2^-108) are formed in plain f32, slowly. A weight below 2^-110
+ * of its row's largest is off by up to 2^-134 of that, and a v below 2^-134
+ * may count as 0. */
 int32_t flk_attn_prefill(const float* q, const float* kcache, const float* vcache, float* o,
                          uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
                          uint32_t n_queries, uint32_t pos0, void* ws, uint64_t ws_bytes);

@@ -522,6 +522,25 @@ EXTREMES = [(16, 8, 1025, 0), (280, 40, 270, 0)]
 
 @pytest.mark.parametrize("d", [128, 64])
 @pytest.mark.parametrize("H,Hkv,nq,pos0", EXTREMES)
+@pytest.mark.parametrize("e", [-120, -117, -110, 95, 117])
+def test_prefill_scores_of_tiny_and_huge_factors(rng, d, H, Hkv, nq, pos0, e):
+    # q * 2^e and k / 2^e have the same scores; with one channel scaled, too.
+    # Rounding alone may differ (f32 scores up to ~6, a weight follows a score's
+    # error): within 2e-6 of the largest output.
+    q = randn(rng, nq * H * d).reshape(nq, H, d)
+    k, v = (randn(rng, nq * Hkv * d).reshape(nq, Hkv, d) for _ in range(2))
+    base = _prefill(q.ravel(), k.ravel(), v.ravel(), H, Hkv, d, nq, pos0)
+    s = np.float32(2.0 ** e)
+    for c in (slice(None), slice(3, 4)):
+        q1, k1 = q.copy(), k.copy()
+        q1[..., c] *= s
+        k1[..., c] /= s
+        got = _prefill(q1.ravel(), k1.ravel(), v.ravel(), H, Hkv, d, nq, pos0)
+        assert np.max(np.abs(got - base)) < 2e-6 * np.abs(base).max(), c
+
+
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("H,Hkv,nq,pos0", EXTREMES)
 @pytest.mark.parametrize("bits", [100, 110, 118])
 def test_prefill_weights_far_below_the_largest(rng, d, H, Hkv, nq, pos0, bits):
     # Key 0 takes nearly all the weight but its v is 0: outputs are what the
