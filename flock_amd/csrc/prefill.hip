@@ -135,13 +135,21 @@ __device__ void row_f32(const PrefillArgs& a, uint32_t lane, const float* qrow, 
 #pragma unroll
     for (int c = 0; c < D / 64; c++) blk[c] = 0.f;
     const uint32_t n = min(key1 - k0, 64u);
-#pragma unroll 8
-    for (uint32_t j = 0; j < n; j++) {
-      const float pj = __builtin_bit_cast(
-          float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), j));
+    for (uint32_t j0 = 0; j0 < n; j0 += 8) {
+      float v[8][D / 64];
 #pragma unroll
-      for (int c = 0; c < D / 64; c++)
-        blk[c] = fmaf(pj, vb[(k0 + j) * stride + 64 * c + lane], blk[c]);
+      for (int j = 0; j < 8; j++)
+#pragma unroll
+        for (int c = 0; c < D / 64; c++)
+          v[j][c] = vb[min(k0 + j0 + j, key1 - 1) * stride + 64 * c + lane];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const float pj = __builtin_bit_cast(
+            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, p), j0 + j));
+#pragma unroll
+        for (int c = 0; c < D / 64; c++)
+          blk[c] = j0 + j < n ? fmaf(pj, v[j][c], blk[c]) : blk[c];
+      }
     }
 #pragma unroll
     for (int c = 0; c < D / 64; c++) acc[c] += blk[c];
@@ -162,10 +170,10 @@ __device__ __forceinline__ float2* ml_lds(uint32x4* const (&buf)[2]) {
 
 // Forms the rows of `s` again, into LDS: channels (divided by l when `final`) and
 // (m, l). Rows that see a NaN in K are NaN already and leave s, so that a NaN token
-// costs little; other rows cost a wave the reads of all their keys, 20 us per 64
-// keys with every CU at it. 16 / 8 heads of 128, us, 2048 and 8192 tokens: 117, 1297;
-// a NaN token half way 138, 1500; an infinite v that every row sees 3480, 82000 (on
-// the f32 kernel, which it does not slow: 157, 2100).
+// costs little; other rows cost a wave the reads of all their keys. 16 / 8 heads of
+// 128, us, 2048 and 8192 tokens: 117, 1270; a NaN token half way 130, 1470; an infinite
+// v that every row sees 2940, 55000 (the f32 kernel, which that does not slow: 157,
+// 2100).
 template <int D>
 __device__ void redo_rows(const PrefillArgs& a, Redo& s, uint32x4* const (&buf)[2], uint32_t kvh,
                           uint32_t qt, uint32_t kt0, uint32_t kt1, bool final) {
