@@ -846,14 +846,17 @@ uint64_t prefill_ws_bytes(const PrefillPlan& p, uint32_t head_dim) {
 }
 
 // Upper bound over every plan with n_queries <= max_queries and pos0 +
-// n_queries <= max_keys: the last max_queries of max_keys positions have the
-// most key tiles, and a cut plan has at most one workgroup for each.
+// n_queries <= max_keys: a cut plan has at most one workgroup for each of a kv
+// head's key tiles, and each of its q tiles at most those of max_keys keys. (The last
+// max_queries positions need not have the most: q tiles that start elsewhere can
+// end in one key tile more.)
 uint64_t prefill_ws_bound(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
                           uint32_t max_queries, uint32_t max_keys) {
-  const PrefillPlan p =
-      prefill_plan(n_heads, n_kv_heads, head_dim, max_queries, max_keys - max_queries);
+  const uint32_t q_per_tile = kRows / (n_heads / n_kv_heads);
+  const uint64_t n_qtiles = ((uint64_t)max_queries + q_per_tile - 1) / q_per_tile;
+  const uint64_t key_tiles = n_qtiles * (((uint64_t)max_keys + kBK - 1) / kBK);
   const uint64_t most = prefill_max_wg(n_kv_heads);
-  const uint64_t wg = p.key_tiles < most ? p.key_tiles : most;
+  const uint64_t wg = key_tiles < most ? key_tiles : most;
   const uint64_t split = split_ws_bytes(wg > 1 ? 2 * wg * n_kv_heads : 0, head_dim);
   const uint64_t small =
       f32::prefill_ws_bound(n_heads, n_kv_heads, head_dim, max_queries, max_keys);

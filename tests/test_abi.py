@@ -159,6 +159,29 @@ def test_workspace_bytes_covers_every_call_in_range():
                 assert 0 <= L.flk_call_workspace_bytes(0, H, Hkv, 128, nk, 0, 1) <= ws
 
 
+def test_workspace_bytes_covers_prefill_calls_of_odd_sizes():
+    # A shorter chunk that ends at the same key can have more key tiles than the
+    # longest one: its q tiles start elsewhere. Drawn sizes, both head widths,
+    # and calls that once needed more than the bound.
+    L = _lib.lib()
+    import random
+    r = random.Random(7)
+    cases = [(48, 8, 64, 235, 235, 211, 24), (32, 4, 64, 315, 315, 276, 39),
+             (7, 1, 128, 704, 702, 687, 17), (40, 8, 128, 265, 243, 205, 60),
+             (24, 3, 128, 363, 363, 339, 24)]
+    for _ in range(20000):
+        hkv = r.choice((1, 2, 3, 4, 5, 8, 16, 40, 100))
+        maxk = r.choice((r.randint(1, 400), r.randint(1, 3000), r.randint(1, 40000)))
+        maxp = r.randint(max(1, maxk - 300), maxk) if r.random() < 0.5 else r.randint(1, min(maxk, 2000))
+        n = max(1, maxp - r.randint(0, 150)) if r.random() < 0.7 else r.randint(1, maxp)
+        pos0 = maxk - n if r.random() < 0.7 else r.randint(0, maxk - n)
+        cases.append((hkv * r.randint(1, 8), hkv, r.choice((64, 128)), maxk, maxp, n, pos0))
+    for H, Hkv, d, maxk, maxp, n, pos0 in cases:
+        ws = L.flk_workspace_bytes(H, Hkv, d, maxk, maxp, 1)
+        need = L.flk_call_workspace_bytes(1, H, Hkv, d, n, pos0, 1)
+        assert need <= ws, (H, Hkv, d, maxk, maxp, n, pos0)
+
+
 def test_ragged_workspace_bound():
     L = _lib.lib()
     for seqs in (1, 3, 64, 200):
