@@ -815,12 +815,13 @@ PrefillPlan prefill_plan(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_di
   const uint64_t least = (p.key_tiles + most - 1) / most;
   const uint64_t rounds = (n_kv_heads + kMaxWG - 1) / kMaxWG;
   const double t0 = head_dim == 128 ? 8.0 : 5.0, t1 = head_dim == 128 ? 5.0 : 2.8;
-  // Runs of whole q tiles end up to a q tile late.
-  const uint64_t whole =
-      p.n_qtiles <= most ? max_kt : (least > max_kt ? least : max_kt) + max_kt / 2;
+  // Runs of whole q tiles end up to a q tile late, but for one run of all.
+  const uint64_t whole = p.n_qtiles <= most ? max_kt
+                         : most == 1        ? p.key_tiles
+                                            : (least > max_kt ? least : max_kt) + max_kt / 2;
   double best = t0 + t1 * rounds * whole;
   p.wg_per_kvh = (uint32_t)(p.n_qtiles < most ? p.n_qtiles : most);
-  for (uint64_t run = least; run <= 4 * least && run < whole; run++) {
+  for (uint64_t run = least; run <= 4 * least && run < whole && run < p.key_tiles; run++) {
     const uint64_t pieces = (max_kt + run - 1) / run + 1;
     const double t = t0 + t1 * rounds * run + 5.0 + 1.3 * ((pieces + 7) / 8);
     if (t < best) {

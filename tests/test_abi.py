@@ -182,6 +182,20 @@ def test_workspace_bytes_covers_prefill_calls_of_odd_sizes():
         assert need <= ws, (H, Hkv, d, maxk, maxp, n, pos0)
 
 
+def test_prefill_of_many_kv_heads_needs_no_partials_of_its_own():
+    # With more than 128 kv heads each has one workgroup, which takes its q tiles
+    # whole: no partials but the f32 kernel's, within the bound.
+    L = _lib.lib()
+    for Hkv in (129, 200, 256, 257, 300):
+        for n, pos0 in ((500, 0), (2000, 0), (64, 4000), (1000, 300)):
+            for g in (1, 4):
+                need = L.flk_call_workspace_bytes(1, Hkv * g, Hkv, 128, n, pos0, 1)
+                ws = L.flk_workspace_bytes(Hkv * g, Hkv, 128, pos0 + n, n, 1)
+                assert need <= ws, (Hkv, g, n, pos0)
+                if n >= 500:
+                    assert need == 0, (Hkv, g, n, pos0)
+
+
 def test_ragged_workspace_bound():
     L = _lib.lib()
     for seqs in (1, 3, 64, 200):
