@@ -107,10 +107,14 @@ uint64_t lm_head_ws_bytes(uint32_t vocab, uint32_t hidden) {
 }
 
 static bool aligned16(const float* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
-// Whether the arrays a[0 .. n) and b[0 .. m) share no memory.
-static bool apart(const float* a, uint32_t n, const float* b, uint32_t m) {
-  const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
-  return pa + 4ull * n <= pb || pb + 4ull * m <= pa;
+// Whether `bytes` at p share no memory with x[0 .. n) and gain[0 .. n).
+static bool apart(const float* x, const float* gain, uint32_t n, const void* p, uint64_t bytes) {
+  const uintptr_t b = reinterpret_cast<uintptr_t>(p);
+  auto off = [&](const float* a) {
+    const uintptr_t pa = reinterpret_cast<uintptr_t>(a);
+    return pa + 4ull * n <= b || b + bytes <= pa;
+  };
+  return off(x) && off(gain);
 }
 
 hipError_t launch_lm_head(const float* x, const float* gain, float eps, const uint8_t* qs,
@@ -122,11 +126,11 @@ hipError_t launch_lm_head(const float* x, const float* gain, float eps, const ui
                                              ws_align(g_max * sizeof(float)));
   // The projection forms the norm itself (one launch less: 151936 x 1024 in an
   // eager loop 42.4 -> 38.6 us) where x and the gain can be read as float4s and
-  // no output lies over them.
+  // nothing that it writes (ws too) lies over them.
   const bool fused = q8_head_norm(vocab, hidden) && aligned16(x) && aligned16(gain) &&
-                     apart(x, hidden, normed, hidden) && apart(gain, hidden, normed, hidden) &&
-                     (logits == nullptr || (apart(x, hidden, logits, vocab) &&
-                                            apart(gain, hidden, logits, vocab)));
+                     apart(x, gain, hidden, normed, 4ull * hidden) &&
+                     apart(x, gain, hidden, ws, lm_head_ws_bytes(vocab, hidden)) &&
+                     (logits == nullptr || apart(x, gain, hidden, logits, 4ull * vocab));
   Q8Fuse fuse;
   hipError_t e = hipSuccess;
   if (fused) {

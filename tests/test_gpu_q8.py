@@ -352,6 +352,31 @@ def test_lm_head_with_the_norm_fused_or_apart(rng, vocab, hidden):
         assert all(np.array_equal(a, b) for a, b in zip(want, other))
 
 
+@pytest.mark.parametrize("inner", ["x", "gain"])
+@pytest.mark.parametrize("vocab,hidden", [(333, 1024), (65537, 1024)])
+def test_lm_head_of_inputs_inside_the_workspace(rng, vocab, hidden, inner):
+    """Workgroups write argmax partials to ws while others still read x and the
+    gain: where those lie inside it, the norm gets a launch of its own."""
+    w = ops.Q8Matrix.from_packed(random_packed(rng, vocab, hidden), vocab, hidden)
+    x = rng.standard_normal(hidden).astype(np.float32)
+    gain = rng.normal(1, 0.1, hidden).astype(np.float32)
+    xb, gb = ops.DeviceBuffer.from_array(x), ops.DeviceBuffer.from_array(gain)
+    ws = ops.DeviceBuffer(ops.lm_head_ws_bytes(vocab, hidden) + 4 * hidden)
+
+    def run(xp, gp):
+        normed, logits = ops.DeviceBuffer(4 * hidden), ops.DeviceBuffer(4 * vocab)
+        ov, oi = ops.DeviceBuffer(4), ops.DeviceBuffer(4)
+        ops.lm_head(xp, gp, oracle.QWEN3_EPS, w, normed, logits, ov, oi, ws)
+        ops.sync()
+        return (normed.download(hidden), logits.download(vocab), ov.download(1),
+                oi.download(1, np.uint32))
+
+    want = run(xb, gb)
+    ws.upload(x if inner == "x" else gain)
+    got = run(ws.ptr if inner == "x" else xb, ws.ptr if inner == "gain" else gb)
+    assert all(np.array_equal(a, b) for a, b in zip(want, got))
+
+
 def test_lm_head_tie_picks_lowest_row(rng):
     vocab, hidden = 151936, 1024
     packed = random_packed(rng, vocab, hidden).reshape(vocab, -1)
