@@ -384,6 +384,12 @@ uint32_t q8_max_workgroups(uint32_t n_rows, uint32_t n_cols);
 // Whether a head's projection forms the norm of x itself (Q8Fuse::normed).
 bool q8_head_norm(uint32_t n_rows, uint32_t n_cols);
 
+// Exported for tests, not part of the ABI: the kernel that a projection of a batch
+// takes. 64 or 32: matrix-core tiles of as many tokens; negative: VALU tiles, as many
+// row tiles per workgroup; 0: the per-token kernels.
+extern "C" int32_t flock_q8_batch_tile(uint32_t n_rows, uint32_t n_cols, uint32_t n_tokens,
+                                       int32_t norm);
+
 // op 0: swiglu(a, b); op 1: a + b (elementwise.wgsl).
 hipError_t launch_elementwise(int op, const float* a, const float* b, float* o, uint32_t n,
                               hipStream_t st);

@@ -1446,6 +1446,8 @@ static Q8MfmaPlan q8_mfma_plan(uint32_t n_rows, uint32_t n_cols, uint32_t n_toke
   // TFLOP/s); the VALU kernels reach 0.75 of that rate.
   double best = 0.95 * (double)n_rows * n_tokens / (64.0 * 64.0 * kSlots) * (78.0 / 58.0);
   Q8MfmaPlan p{0, 0};
+  // A tile's 64 rows of x lie within 4 GiB (32-bit byte offsets).
+  if (n_tokens < 64 || n_cols > 1u << 24) return p;
   for (uint32_t nt = 2; nt <= 4; nt += 2) {
     const uint64_t n_tt = (n_tokens + 16 * nt - 1) / (16 * nt);
     const uint64_t tiles = n_rt * n_tt;
@@ -1460,6 +1462,25 @@ static Q8MfmaPlan q8_mfma_plan(uint32_t n_rows, uint32_t n_cols, uint32_t n_toke
     }
   }
   return p;
+}
+
+// Row tiles per workgroup of the VALU tile kernels (rows of one chunk): as many as
+// keep the grid at kMmMinWorkgroups or more, up to kMmRowTiles.
+static uint32_t q8_row_tiles(uint32_t n_rows, uint32_t n_cols, uint32_t n_tokens) {
+  const uint32_t n_rt = (n_rows + kMmRows - 1) / kMmRows;
+  const uint32_t n_tt = (n_tokens + kMmTokens - 1) / kMmTokens;
+  uint32_t rpw = 1;
+  while (n_cols <= (uint32_t)kMmChunkCols && rpw < kMmRowTiles &&
+         (uint64_t)((n_rt + 2 * rpw - 1) / (2 * rpw)) * n_tt >= kMmMinWorkgroups)
+    rpw *= 2;
+  return rpw;
+}
+
+extern "C" int32_t flock_q8_batch_tile(uint32_t n_rows, uint32_t n_cols, uint32_t n_tokens,
+                                       int32_t norm) {
+  if (n_rows == 0 || n_cols == 0 || n_tokens < FLK_Q8_MM_MIN_TOKENS) return 0;
+  const Q8MfmaPlan p = q8_mfma_plan(n_rows, n_cols, n_tokens, norm != 0);
+  return p.nt != 0 ? (int32_t)(16 * p.nt) : -(int32_t)q8_row_tiles(n_rows, n_cols, n_tokens);
 }
 
 // Workgroups: one resident wave of them (every CU filled to its occupancy
@@ -1587,14 +1608,9 @@ hipError_t launch_q8_matvec(const uint8_t* qs, const uint16_t* scales, const flo
   const uint32_t n_rt = (n_rows + kMmRows - 1) / kMmRows;
   const uint32_t n_tt = (n_tokens + kMmTokens - 1) / kMmTokens;
   const bool one = n_cols <= (uint32_t)kMmChunkCols;
-  // Row tiles per workgroup (rows of one chunk): as many as keep the grid at
-  // kMmMinWorkgroups or more, up to kMmRowTiles.
-  uint32_t rpw = 1;
-  while (one && rpw < kMmRowTiles && (uint64_t)((n_rt + 2 * rpw - 1) / (2 * rpw)) * n_tt >=
-                                          kMmMinWorkgroups)
-    rpw *= 2;
+  const uint32_t rpw = q8_row_tiles(n_rows, n_cols, n_tokens);
   const uint32_t n_rg = (n_rt + rpw - 1) / rpw;
-  const Q8MfmaPlan mp = n_tokens >= 64 && best_val == nullptr
+  const Q8MfmaPlan mp = best_val == nullptr
                             ? q8_mfma_plan(n_rows, n_cols, n_tokens, a.norm_gain != nullptr)
                             : Q8MfmaPlan{0, 0};
   if (mp.nt != 0) {

@@ -319,3 +319,14 @@ def test_prefill_rejects_rows_too_wide_for_its_tile_offsets():
     rc, msg = code_and_msg(L.flk_attn_prefill(FAKE, FAKE, FAKE, FAKE, 65536, 65536, 128, 4, 0,
                                               FAKE, 1 << 40))
     assert rc == _lib.FLK_ERR_UNSUPPORTED and "2 GiB" in msg
+
+
+def test_matrix_core_tiles_take_only_rows_their_offsets_reach():
+    # 64 rows of x are addressed with 32-bit byte offsets: 2^24 columns are the
+    # widest (63 rows of them are 64 MiB short of 4 GiB).
+    L = _lib.lib()
+    assert L.flock_q8_batch_tile(4096, 1024, 2048, 0) == 64
+    for cols, tile in ((1 << 24, 64), ((1 << 24) + 32, -1), (1 << 26, -1)):
+        assert L.flock_q8_batch_tile(4096, cols, 2048, 0) == tile, cols
+    assert L.flock_q8_batch_tile(4096, 1024, 63, 0) < 0
+    assert L.flock_q8_batch_tile(4096, 1024, 7, 0) == 0
