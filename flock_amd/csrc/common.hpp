@@ -321,6 +321,11 @@ hipError_t launch_prefill(const float* q, const float* kcache, const float* vcac
                           uint32_t n_queries, uint32_t pos0, const PrefillPlan& p, void* ws,
                           hipStream_t st);
 
+// Exported for tests, not part of the ABI: how a valid call's work is dealt out. 0:
+// the f32 kernel; 1: a workgroup per q tile; 2: runs of whole q tiles; 3: cut ones.
+extern "C" int32_t flock_prefill_schedule(uint32_t n_heads, uint32_t n_kv_heads,
+                                          uint32_t head_dim, uint32_t n_queries, uint32_t pos0);
+
 // ------------------------------------------------------------------ argmax --
 // argmax.wgsl's contract: (va, ia) beats (vb, ib) if va > vb, or va == vb and
 // ia < ib; the empty result is (-3.4028235e38, 0xffffffff), and a NaN never

@@ -836,6 +836,13 @@ PrefillPlan prefill_plan(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_di
   return p;
 }
 
+extern "C" int32_t flock_prefill_schedule(uint32_t n_heads, uint32_t n_kv_heads,
+                                          uint32_t head_dim, uint32_t n_queries, uint32_t pos0) {
+  const PrefillPlan p = prefill_plan(n_heads, n_kv_heads, head_dim, n_queries, pos0);
+  if (p.use_small) return 0;
+  return p.cut ? 3 : p.n_qtiles == p.wg_per_kvh ? 1 : 2;
+}
+
 static uint64_t split_ws_bytes(uint64_t slots, uint32_t head_dim) {
   if (slots == 0) return 0;
   return ws_align(slots * kRows * sizeof(float2)) + slots * kRows * head_dim * sizeof(float);

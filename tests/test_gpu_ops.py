@@ -395,17 +395,7 @@ def test_prefill_groups_5_6_7(rng, d, H, Hkv, nq, pos0):
     assert meets_bar(m), fmt(m)
 
 
-# (heads, kv heads, queries, pos0) of enough work for the split kernel, at the
-# edges of its 128-row q tiles, its 64-key tiles and the equal runs of key tiles
-# that workgroups take: whole and cut q tiles, runs that start and end inside
-# them, kv heads that 256 workgroups do not divide by, q tiles left partly
-# empty, MHA and MQA.
-@pytest.mark.parametrize("d", [128, 64])
-@pytest.mark.parametrize("H,Hkv,nq,pos0", [
-    (16, 8, 1025, 0), (16, 8, 960, 64), (16, 8, 513, 448), (5, 5, 1537, 0), (5, 5, 513, 2500),
-    (8, 1, 1100, 130), (24, 3, 600, 511), (40, 40, 300, 0), (56, 8, 257, 1000),
-])
-def test_prefill_schedule_edges(rng, d, H, Hkv, nq, pos0):
+def _check_prefill(rng, d, H, Hkv, nq, pos0):
     nk = pos0 + nq
     q = randn(rng, nq * H * d)
     k, v = randn(rng, nk * Hkv * d), randn(rng, nk * Hkv * d)
@@ -417,6 +407,34 @@ def test_prefill_schedule_edges(rng, d, H, Hkv, nq, pos0):
     # growing like their square root, within 64 roundings of the largest output
     # (near-zero outputs make relative bounds depend on the draw).
     assert m["gpu_abs_vs_f64"] < 64 * 2.0 ** -24 * np.abs(want).max(), fmt(m)
+
+
+# (heads, kv heads, queries, pos0) of enough work for the split kernel, at the
+# edges of its 128-row q tiles, its 64-key tiles and the equal runs of key tiles
+# that workgroups take: runs that start and end inside q tiles and hold whole ones,
+# kv heads that 256 workgroups do not divide by, q tiles left partly empty, MHA and
+# MQA.
+@pytest.mark.parametrize("d", [128, 64])
+@pytest.mark.parametrize("H,Hkv,nq,pos0", [
+    (16, 8, 1025, 0), (16, 8, 960, 64), (16, 8, 513, 448), (5, 5, 1537, 0), (5, 5, 513, 2500),
+    (8, 1, 1100, 130), (24, 3, 600, 511), (40, 40, 300, 0), (56, 8, 257, 1000),
+])
+def test_prefill_schedule_edges(rng, d, H, Hkv, nq, pos0):
+    assert ops.lib().flock_prefill_schedule(H, Hkv, d, nq, pos0) == 3  # cut q tiles
+    _check_prefill(rng, d, H, Hkv, nq, pos0)
+
+
+# Calls whose q tiles stay whole: one for each workgroup (schedule 1) or runs of
+# them (2), with up to one workgroup for each of more kv heads than CUs.
+@pytest.mark.parametrize("d,H,Hkv,nq,pos0,schedule", [
+    (128, 448, 64, 70, 512, 1), (64, 448, 64, 70, 512, 1), (128, 300, 300, 1, 97, 1),
+    (64, 771, 257, 1, 103, 1), (128, 256, 256, 33, 342, 1),
+    (64, 280, 40, 270, 0, 2), (128, 258, 129, 65, 0, 2), (64, 390, 65, 65, 0, 2),
+    (64, 1542, 257, 41, 0, 2), (128, 400, 200, 150, 65, 2),
+])
+def test_prefill_of_whole_q_tiles(rng, d, H, Hkv, nq, pos0, schedule):
+    assert ops.lib().flock_prefill_schedule(H, Hkv, d, nq, pos0) == schedule
+    _check_prefill(rng, d, H, Hkv, nq, pos0)
 
 
 @pytest.mark.parametrize("d", [128, 64])

@@ -168,17 +168,38 @@ def test_tile_kernels_equal_per_token_kernel_on_random_shapes():
         assert np.array_equal(big, small), (case, rows, cols, n, fuse)
 
 
-@pytest.mark.parametrize("rows,cols,n,fuse", [
-    (4096, 1024, 1000, "norm"),      # 64 x 64 tiles, one block per leaf, ragged last tokens
-    (6144, 1024, 500, "gate_up"),    # 64 x 32 tiles
-    (4097, 256, 601, "up"),          # 8 leaves; one row in the last row tile
-    (4100, 96, 700, "plain"),        # fewer blocks than the 8 leaves written out
-    (2050, 2080, 1100, "res"),       # 65 blocks: one leaf of two
-    (1000, 3072, 2100, "norm"),      # leaves of two blocks and of one; runs cross token tiles
+# Every instance of q8_mfma_kernel: 32 and 64 tokens per tile, the three input
+# fusions, one block per leaf of the tree (8, 16, 32 or 64 blocks per row) and the
+# general walk; one row in the last row tile wherever the plan allows it.
+@pytest.mark.parametrize("rows,cols,n,fuse,tile", [
+    (513, 256, 1696, "plain", 32),
+    (513, 2080, 1696, "res", 32),     # 65 blocks: one leaf of two
+    (704, 1024, 1236, "up", 32),
+    (513, 2080, 1696, "up", 32),
+    (1473, 1024, 1945, "norm", 32),
+    (961, 2080, 1944, "norm", 32),
+    (4096, 1024, 1000, "norm", 32),
+    (6144, 1024, 500, "gate_up", 32),
+    (4100, 96, 700, "plain", 32),     # fewer blocks than the 8 leaves written out
+    (1537, 1024, 1068, "res", 64),
+    (1537, 96, 1068, "plain", 64),
+    (1537, 4224, 1068, "plain", 64),  # leaves of two and of three blocks
+    (1537, 1024, 1068, "up", 64),
+    (832, 3072, 1973, "up", 64),
+    (1024, 3072, 2048, "res", 64),    # a layer's down projection
+    (3457, 1024, 2108, "norm", 64),
+    (6144, 1024, 2048, "gate_up", 64),
+    (2497, 2080, 1457, "norm", 64),
+    # And the VALU tiles: few and many row tiles per workgroup, rows past a tile.
+    (4097, 256, 601, "up", -8),
+    (4096, 1024, 777, "norm", -8),
+    (2050, 2080, 1100, "res", -1),
+    (1000, 3072, 2100, "norm", -1),
 ])
-def test_matrix_core_tiles_match_small_batches(rng, rows, cols, n, fuse):
+def test_matrix_core_tiles_match_small_batches(rng, rows, cols, n, fuse, tile):
     """Batches that fill the GPU with 64-row tiles (q8_mfma_kernel) equal the
     same tokens projected 7 at a time (the per-token kernel), bit for bit."""
+    assert ops.lib().flock_q8_batch_tile(rows, cols, n, fuse in ("norm", "gate_up")) == tile
     w = ops.Q8Matrix.from_packed(random_packed(rng, rows, cols), rows, cols)
     x = rng.standard_normal((n, cols)).astype(np.float32)
     x[:, 3] *= 1e-39  # subnormal products

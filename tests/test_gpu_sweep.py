@@ -113,7 +113,25 @@ def test_decode_shape_sweep(rng, H, Hkv, d, nk):
     assert ok, (fmt(m), ties)
 
 
-@pytest.mark.parametrize("H,Hkv,d,nq,pos0", _prefill_cases(20))
+def _split_prefill_cases(n: int, seed: int = 20261206, max_flop: float = 3e9):
+    """Shapes that the split kernel takes (the draws above are too small for it)."""
+    r = np.random.default_rng(seed)
+    out = []
+    while len(out) < n:
+        hkv = int(r.choice(KV_HEADS + (20, 70, 130)))
+        g = int(r.integers(1, 9))
+        d = int(r.choice((64, 128)))
+        nq = int(r.integers(20, 900))
+        pos0 = int(r.choice((0, 1, 63, 64, 65))) if r.random() < 0.5 else int(r.integers(0, 3001))
+        if 4 * hkv * g * d * (nq * pos0 + nq * (nq + 1) // 2) > max_flop:
+            continue
+        if ops.lib().flock_prefill_schedule(hkv * g, hkv, d, nq, pos0) == 0:
+            continue
+        out.append((hkv * g, hkv, d, nq, pos0))
+    return out
+
+
+@pytest.mark.parametrize("H,Hkv,d,nq,pos0", _prefill_cases(20) + _split_prefill_cases(20))
 def test_prefill_shape_sweep(rng, H, Hkv, d, nq, pos0):
     nk = pos0 + nq
     q = randn(rng, nq * H * d)
