@@ -380,7 +380,6 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo*
   // The row's q, pre-multiplied by scale * log2(e) so that S^T comes out in
   // base-2 units, split.
   uint32x4 qf[NG][3];
-  uint32_t q_mid = ~0u;  // bits 14 and 30: every element's top two exponent bits differ
 #pragma unroll
   for (int j = 0; j < NG; j++) {
     const float4 x = p.q[2 * j], y = p.q[2 * j + 1];
@@ -391,11 +390,23 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo*
       split_pair(e[2 * i] * a.scale_log2e, e[2 * i + 1] * a.scale_log2e, u);
 #pragma unroll
       for (int k = 0; k < 3; k++) qf[j][k][i] = u[k];
-      q_mid &= u[0] ^ (u[0] << 1);
     }
   }
+  lds_barrier();  // before the branch below, or every wave waits for the slowest q
   // 2^-63 <= |q| < 2^65 has top exponent bits 01 or 10; a row with others (or
-  // zeros) is read again and looked at.
+  // zeros) is read again and looked at. Each of the row's two waves takes half of q.
+  uint32_t q_mid = ~0u;  // bits 14 and 30: the top two exponent bits differ everywhere
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+    if (h == half) {  // uniform
+#pragma unroll
+      for (int j = 0; j < NG / 2; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const uint32_t u = qf[h * NG / 2 + j][0][i];
+          q_mid &= u ^ (u << 1);
+        }
+    }
   bool q_out = false;
   if (__builtin_amdgcn_ballot_w64((q_mid & 0x40004000u) != 0x40004000u) != 0) {  // uniform
     float4 q[D / 8];
@@ -413,7 +424,6 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo*
     }
     q_out = least < kTinyQ || !(most < kLargeQ);
   }
-  lds_barrier();
 
   floatx16 oacc[CB];
 #pragma unroll
@@ -585,78 +595,67 @@ __device__ __forceinline__ void run_item(const PrefillArgs& a, Pipe<D>& p, Redo*
   const float w1 = __builtin_amdgcn_exp2f(m_run - M);
   const float w2 = __builtin_amdgcn_exp2f(ml2.x - M);
   const float L = l_run * w1 + ml2.y * w2;
+  // Stored as they come, and looked at meanwhile: stores held back until all were
+  // looked at cost 0.5 us per item.
+  float* dst;
+  if (final) {
+    dst = a.o + row.offset(a);
+  } else {
+    dst = a.part_acc + (slot * kRows + r) * D;
+    if (lg == 0 && half == 0) a.part_ml[slot * kRows + r] = make_float2(M, L);
+  }
+  dst += 32 * HB * half + 4 * lg;  // channel 32c + 8j of this lane at 32c + 8j
+  float least = INFINITY, most = 0.f;  // magnitudes; a NaN stays in `most`
 #pragma unroll
   for (int c = 0; c < HB; c++)
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       const float4 x = __builtin_bit_cast(
           float4, (half ? bv : bn)[(((wave & 3) * HB + c) * 4 + j) * 64 + lane]);
-      mine[c][4 * j] = mine[c][4 * j] * w1 + x.x * w2;
-      mine[c][4 * j + 1] = mine[c][4 * j + 1] * w1 + x.y * w2;
-      mine[c][4 * j + 2] = mine[c][4 * j + 2] * w1 + x.z * w2;
-      mine[c][4 * j + 3] = mine[c][4 * j + 3] * w1 + x.w * w2;
-    }
-  if (final) {  // uniform
+      float4 v = make_float4(mine[c][4 * j] * w1 + x.x * w2, mine[c][4 * j + 1] * w1 + x.y * w2,
+                             mine[c][4 * j + 2] * w1 + x.z * w2,
+                             mine[c][4 * j + 3] * w1 + x.w * w2);
+      if (final) v = make_float4(v.x / L, v.y / L, v.z / L, v.w / L);
+      const float e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-    for (int c = 0; c < HB; c++)
-#pragma unroll
-      for (int i = 0; i < 16; i++) mine[c][i] = mine[c][i] / L;
-  }
-  float least = INFINITY, most = 0.f;  // magnitudes; a NaN stays in `most`
-#pragma unroll
-  for (int c = 0; c < HB; c++)
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-      least = fminf(least, fabsf(mine[c][i]));
-      most = __builtin_elementwise_maximum(most, fabsf(mine[c][i]));
+      for (int i = 0; i < 4; i++) {
+        least = fminf(least, fabsf(e[i]));
+        most = __builtin_elementwise_maximum(most, fabsf(e[i]));
+      }
+      if (row_ok || !final) *reinterpret_cast<float4*>(dst + 32 * c + 8 * j) = v;
     }
   const float tiny = final ? kTinyOutput : kTinyOutput * L;
-  bool again = row_ok && (q_out || !(most < INFINITY) || !(least >= tiny));
-  if (__builtin_amdgcn_ballot_w64(again) != 0) {  // uniform
+  const bool look = row_ok && (q_out || !(most < INFINITY) || !(least >= tiny));
+  if (__builtin_amdgcn_ballot_w64(look) != 0) {  // uniform
     least = INFINITY;  // of the others than 0
 #pragma unroll
     for (int c = 0; c < HB; c++)
 #pragma unroll
-      for (int i = 0; i < 16; i++)
-        least = fminf(least, mine[c][i] != 0.f ? fabsf(mine[c][i]) : INFINITY);
-    again = row_ok && (q_out || !(most < INFINITY) || least < tiny);
-    if (again) {
+      for (int j = 0; j < 4; j++) {
+        const float4 v = *reinterpret_cast<const float4*>(dst + 32 * c + 8 * j);
+        const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) least = fminf(least, e[i] != 0.f ? fabsf(e[i]) : INFINITY);
+      }
+    if (row_ok && (q_out || !(most < INFINITY) || least < tiny)) {
       atomicOr(&redo->bad[wave & 3], 1u << lc);
       redo->any = 1;
     }
   }
-  auto store = [&](float2 ml) {
-    float* dst;
-    if (final) {
-      dst = a.o + row.offset(a);
-    } else {
-      dst = a.part_acc + (slot * kRows + r) * D;
-      if (lg == 0 && half == 0) a.part_ml[slot * kRows + r] = ml;
-    }
-#pragma unroll
-    for (int c = 0; c < HB; c++)
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-        *reinterpret_cast<float4*>(dst + 32 * (HB * half + c) + 8 * j + 4 * lg) =
-            make_float4(mine[c][4 * j], mine[c][4 * j + 1], mine[c][4 * j + 2],
-                        mine[c][4 * j + 3]);
-  };
-  if (!again && (row_ok || !final)) store(make_float2(M, L));
   __syncthreads();  // every wave is done with the exchange (the next item's V goes there)
   if (redo->any) {  // uniform
     uint32x4* const buf[2] = {bv, bn};
     redo_rows<D>(a, *redo, buf, kvh, qt, kt0, kt1, final);
-    float2 ml = make_float2(M, L);
-    if (redo->bad[wave & 3] >> lc & 1) {  // also where this lane's channels are stored
-      again = true;
+    if (redo->bad[wave & 3] >> lc & 1) {
       const float* x = row_lds<D>(buf, r) + 32 * HB * half + 4 * lg;
 #pragma unroll
       for (int c = 0; c < HB; c++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) mine[c][i] = x[32 * c + 8 * (i / 4) + i % 4];
-      ml = ml_lds<D>(buf)[r];
+        for (int j = 0; j < 4; j++)
+          *reinterpret_cast<float4*>(dst + 32 * c + 8 * j) =
+              *reinterpret_cast<const float4*>(x + 32 * c + 8 * j);
+      if (!final && lg == 0 && half == 0) a.part_ml[slot * kRows + r] = ml_lds<D>(buf)[r];
     }
-    if (again) store(ml);
     // Requested again, so that nothing else is held over redo_rows.
     QRow<D>(a, kvh, nxt_qt).fetch(p.q, a);
     ld.load_v(st, a, kvh, nxt_kt);
