@@ -50,6 +50,11 @@ static int32_t check_heads(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_
   return FLK_OK;
 }
 
+static bool ws_holds(const void* ws, uint64_t ws_bytes, uint64_t need) {
+  return need == 0 || (ws != nullptr && ws_bytes >= need &&
+                       reinterpret_cast<uintptr_t>(ws) % 256 == 0);
+}
+
 static int32_t check_ws(void* ws, uint64_t ws_bytes, uint64_t need) {
   if (need == 0) return FLK_OK;  // single-split launch: no partials
   if (ws == nullptr || ws_bytes < need)
@@ -333,12 +338,18 @@ int32_t flk_attn_prefill(const float* q, const float* kcache, const float* vcach
                 n_kv_heads, head_dim);
   PrefillPlan p = prefill_plan(n_heads, n_kv_heads, head_dim, n_queries, pos0);
   // A workspace that holds the f32 kernel's partials (none for many q tiles) is
-  // enough: the call then takes that kernel.
-  rc = check_ws(ws, ws_bytes, prefill_ws_bytes(p, head_dim));
-  if (rc && !p.use_small) {
-    p.use_small = true;
-    rc = check_ws(ws, ws_bytes, prefill_ws_bytes(p, head_dim));
+  // enough: the call then takes that kernel. So does one in place (o over q) where it
+  // can: the split kernel reads a row of q again, after it has stored the row's output,
+  // if it forms the row anew.
+  const uint64_t row_bytes = 4ull * n_heads * head_dim * n_queries;
+  const uintptr_t qa = reinterpret_cast<uintptr_t>(q), oa = reinterpret_cast<uintptr_t>(o);
+  const bool in_place = qa < oa + row_bytes && oa < qa + row_bytes;
+  if (!p.use_small && (in_place || !ws_holds(ws, ws_bytes, prefill_ws_bytes(p, head_dim)))) {
+    PrefillPlan small = p;
+    small.use_small = true;
+    if (ws_holds(ws, ws_bytes, prefill_ws_bytes(small, head_dim))) p = small;
   }
+  rc = check_ws(ws, ws_bytes, prefill_ws_bytes(p, head_dim));
   if (rc) return rc;
   return hip_status(launch_prefill(q, kcache, vcache, o, n_heads, n_kv_heads, head_dim, n_queries,
                                    pos0, p, ws, g_stream),

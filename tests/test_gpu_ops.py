@@ -534,6 +534,25 @@ def test_prefill_rows_keep_their_bits_beside_others_that_are_not_finite(rng, d, 
     assert np.all(np.isnan(got[at, 0])) and np.all(np.isnan(got[at:, 8:10]))
 
 
+@pytest.mark.parametrize("d", [128, 64])
+def test_prefill_in_place(rng, d):
+    # o over q: rows that are formed anew (here: two of infinite q) need their q. Both
+    # kernels are within 64 eps of the exact value (as without a workspace, above).
+    H, Hkv, nq = 16, 8, 1025
+    q = randn(rng, nq * H * d).reshape(nq, H, d)
+    k, v = randn(rng, nq * Hkv * d), randn(rng, nq * Hkv * d)
+    q[:, 4, 0] *= np.float32(2.0 ** -120)
+    q[30, 2] = q[700, 2] = np.inf
+    k[:] = np.abs(k)
+    want = _prefill(q.ravel(), k, v, H, Hkv, d, nq, 0).reshape(nq, H, d)
+    qo = dev(q.ravel())
+    ops.attn_prefill(qo, dev(k), dev(v), qo, H, Hkv, d, nq, 0, ops.Workspace(H, Hkv, d, nq, nq))
+    got = get(qo, nq * H * d).reshape(nq, H, d)
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan) and nan[30, 2].all() and nan.sum() == 2 * d
+    assert np.max(np.abs((got - want)[~nan])) < 2 * 64 * 2.0 ** -24 * np.abs(want[~nan]).max()
+
+
 # (heads, kv heads, queries, pos0): cut q tiles, and whole ones.
 EXTREMES = [(16, 8, 1025, 0), (280, 40, 270, 0)]
 
