@@ -773,9 +773,20 @@ static uint64_t prefill_max_wg(uint32_t n_kv_heads) {
 
 // Estimated time (us) of the f32 kernel under its plan: 1-tile items cost 5 +
 // 4.4 (head_dim 64: 3.5 + 2.5), a merge 5; more workgroups than CUs run in rounds.
+// With more kv heads than half the CUs, pairs of q tiles are counted more closely
+// (the middle one of an odd number runs alone) and every round of one workgroup per
+// CU (head_dim 128) starts anew.
 static double small_us(const f32::PrefillPlan& p, uint32_t n_kv_heads, uint32_t head_dim,
                        uint32_t n_queries, uint32_t pos0) {
   uint64_t wg = 0, run = 0;
+  if (p.paired && prefill_max_wg(n_kv_heads) == 1) {
+    const bool one = p.n_qtiles == 1;
+    run = qtile_kt(p.n_qtiles - 1, p.q_per_tile, n_queries, pos0) +
+          (one ? 0 : qtile_kt(0, p.q_per_tile, n_queries, pos0));
+    const uint64_t halves = (uint64_t)n_kv_heads * (one ? 2 : p.n_qtiles);
+    const double rounds = (double)((halves + 2 * kMaxWG - 1) / (2 * kMaxWG));
+    return head_dim == 128 ? rounds * (5.0 + 4.4 * run) : 3.5 + 2.5 * rounds * run;
+  }
   if (p.paired) {
     wg = p.work_per_kvh;
     run = qtile_kt(p.n_qtiles - 1, p.q_per_tile, n_queries, pos0) +
@@ -814,11 +825,12 @@ PrefillPlan prefill_plan(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_di
   const uint64_t least = (p.key_tiles + most - 1) / most;
   const uint64_t rounds = (n_kv_heads + kMaxWG - 1) / kMaxWG;
   const double t0 = head_dim == 128 ? 8.0 : 5.0, t1 = head_dim == 128 ? 5.0 : 2.8;
-  // Runs of whole q tiles end up to a q tile late, but for one run of all.
-  const uint64_t whole = p.n_qtiles <= most ? max_kt
-                         : most == 1        ? p.key_tiles
-                                            : (least > max_kt ? least : max_kt) + max_kt / 2;
-  double best = t0 + t1 * rounds * whole;
+  // Runs of whole q tiles end up to a q tile late; one run of all does not, and its
+  // further q tiles cost 3 each.
+  const uint64_t whole =
+      p.n_qtiles <= most ? max_kt : (least > max_kt ? least : max_kt) + max_kt / 2;
+  double best = most == 1 ? rounds * (t0 + 3.0 * (p.n_qtiles - 1) + t1 * p.key_tiles)
+                          : t0 + t1 * rounds * whole;
   p.wg_per_kvh = (uint32_t)(p.n_qtiles < most ? p.n_qtiles : most);
   for (uint64_t run = least; run <= 4 * least && run < whole && run < p.key_tiles; run++) {
     const uint64_t pieces = (max_kt + run - 1) / run + 1;
@@ -831,7 +843,8 @@ PrefillPlan prefill_plan(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_di
   }
   p.partial_slots = p.cut ? 2ull * p.wg_per_kvh * n_kv_heads : 0;
   p.small = f32::prefill_plan(n_heads, n_kv_heads, head_dim, n_queries, pos0);
-  p.use_small = small_us(p.small, n_kv_heads, head_dim, n_queries, pos0) < 1.3 * best;
+  p.use_small = small_us(p.small, n_kv_heads, head_dim, n_queries, pos0) <
+                (most == 1 ? 1.1 : 1.3) * best;
   return p;
 }
 

@@ -196,6 +196,16 @@ def test_prefill_of_many_kv_heads_needs_no_partials_of_its_own():
                     assert need == 0, (Hkv, g, n, pos0)
 
 
+def test_short_chunks_of_many_kv_heads_take_the_f32_kernel():
+    # Two rounds of workgroups with one or two short q tiles each: the f32 kernel's
+    # smaller items are done sooner (a third, measured).
+    L = _lib.lib()
+    for H, Hkv, d, n, pos0 in [(300, 300, 128, 1, 97), (771, 257, 64, 1, 103),
+                               (256, 256, 128, 33, 342), (1542, 257, 64, 41, 0),
+                               (258, 129, 128, 65, 0), (1200, 200, 64, 106, 0)]:
+        assert L.flock_prefill_schedule(H, Hkv, d, n, pos0) == 0, (H, Hkv, d, n, pos0)
+
+
 def test_ragged_workspace_bound():
     L = _lib.lib()
     for seqs in (1, 3, 64, 200):

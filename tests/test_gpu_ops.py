@@ -427,10 +427,10 @@ def test_prefill_schedule_edges(rng, d, H, Hkv, nq, pos0):
 # Calls whose q tiles stay whole: one for each workgroup (schedule 1) or runs of
 # them (2), with up to one workgroup for each of more kv heads than CUs.
 @pytest.mark.parametrize("d,H,Hkv,nq,pos0,schedule", [
-    (128, 448, 64, 70, 512, 1), (64, 448, 64, 70, 512, 1), (128, 300, 300, 1, 97, 1),
-    (64, 771, 257, 1, 103, 1), (128, 256, 256, 33, 342, 1),
-    (64, 280, 40, 270, 0, 2), (128, 258, 129, 65, 0, 2), (64, 390, 65, 65, 0, 2),
-    (64, 1542, 257, 41, 0, 2), (128, 400, 200, 150, 65, 2),
+    (128, 448, 64, 70, 512, 1), (64, 448, 64, 70, 512, 1), (128, 600, 200, 39, 50, 1),
+    (64, 256, 256, 119, 3, 1), (128, 640, 160, 1, 700, 1),
+    (64, 280, 40, 270, 0, 2), (128, 800, 160, 39, 0, 2), (64, 390, 65, 65, 0, 2),
+    (128, 1200, 400, 79, 31, 2), (64, 2400, 400, 21, 0, 1), (64, 2400, 400, 33, 57, 2),
 ])
 def test_prefill_of_whole_q_tiles(rng, d, H, Hkv, nq, pos0, schedule):
     assert ops.lib().flock_prefill_schedule(H, Hkv, d, nq, pos0) == schedule
