@@ -773,34 +773,37 @@ static uint64_t prefill_max_wg(uint32_t n_kv_heads) {
 
 // Estimated time (us) of the f32 kernel under its plan: 1-tile items cost 5 +
 // 4.4 (head_dim 64: 3.5 + 2.5), a merge 5; more workgroups than CUs run in rounds.
-// With more kv heads than half the CUs, pairs of q tiles are counted more closely
-// (the middle one of an odd number runs alone) and every round of one workgroup per
-// CU (head_dim 128) starts anew.
+// Closer where that is known to mislead, at head_dim 128 (one workgroup per CU) and
+// with more kv heads than half the CUs: pairs of q tiles count by their halves (the
+// middle one of an odd number runs alone); at head_dim 128 whole q tiles of a second
+// round start where the lightest of the first end.
 static double small_us(const f32::PrefillPlan& p, uint32_t n_kv_heads, uint32_t head_dim,
                        uint32_t n_queries, uint32_t pos0) {
-  uint64_t wg = 0, run = 0;
-  if (p.paired && prefill_max_wg(n_kv_heads) == 1) {
-    const bool one = p.n_qtiles == 1;
-    run = qtile_kt(p.n_qtiles - 1, p.q_per_tile, n_queries, pos0) +
-          (one ? 0 : qtile_kt(0, p.q_per_tile, n_queries, pos0));
-    const uint64_t halves = (uint64_t)n_kv_heads * (one ? 2 : p.n_qtiles);
-    const double rounds = (double)((halves + 2 * kMaxWG - 1) / (2 * kMaxWG));
-    return head_dim == 128 ? rounds * (5.0 + 4.4 * run) : 3.5 + 2.5 * rounds * run;
-  }
+  const double t0 = head_dim == 128 ? 5.0 : 3.5, t1 = head_dim == 128 ? 4.4 : 2.5;
+  const bool many = prefill_max_wg(n_kv_heads) == 1;
+  auto size = [&](uint32_t qt) {
+    return (uint64_t)qtile_kt(qt, p.q_per_tile, n_queries, pos0);
+  };
+  const uint64_t heaviest = size(p.n_qtiles - 1);
   if (p.paired) {
-    wg = p.work_per_kvh;
-    run = qtile_kt(p.n_qtiles - 1, p.q_per_tile, n_queries, pos0) +
-          qtile_kt(0, p.q_per_tile, n_queries, pos0);
-  } else {
-    run = p.ktiles_per_split;
-    for (uint32_t qt = 0; qt < p.n_qtiles; qt++)
-      wg += (qtile_kt(qt, p.q_per_tile, n_queries, pos0) + run - 1) / run;
-    const uint64_t heaviest = qtile_kt(p.n_qtiles - 1, p.q_per_tile, n_queries, pos0);
-    if (run > heaviest) run = heaviest;
+    const uint64_t run = heaviest + (many && p.n_qtiles == 1 ? 0 : size(0));
+    uint64_t halves = 2ull * p.work_per_kvh;
+    if ((many || head_dim == 128) && p.n_qtiles > 1) halves = p.n_qtiles;
+    const double rounds = (double)((halves * n_kv_heads + 2 * kMaxWG - 1) / (2 * kMaxWG));
+    return many && head_dim == 128 ? rounds * (t0 + t1 * run) : t0 + t1 * rounds * run;
   }
+  if (head_dim == 128 && !many && p.max_splits == 1 && p.n_qtiles * n_kv_heads > kMaxWG) {
+    const uint32_t last = (kMaxWG - 1) / n_kv_heads, next = kMaxWG / n_kv_heads;
+    const double one = t0 + t1 * heaviest;
+    const double two =
+        2 * t0 + t1 * (size(p.n_qtiles - 1 - last) + size(p.n_qtiles - 1 - next));
+    return one > two ? one : two;
+  }
+  uint64_t wg = 0, run = p.ktiles_per_split;
+  for (uint32_t qt = 0; qt < p.n_qtiles; qt++) wg += (size(qt) + run - 1) / run;
+  if (run > heaviest) run = heaviest;
   const double rounds = (double)((wg * n_kv_heads + kMaxWG - 1) / kMaxWG);
-  const double tiles = rounds * run;
-  return (head_dim == 128 ? 5.0 + 4.4 * tiles : 3.5 + 2.5 * tiles) + (p.max_splits > 1 ? 5.0 : 0.0);
+  return t0 + t1 * rounds * run + (p.max_splits > 1 ? 5.0 : 0.0);
 }
 
 // A kv head's q tiles either stay whole, one workgroup each (or, with more of
@@ -808,11 +811,15 @@ static double small_us(const f32::PrefillPlan& p, uint32_t n_kv_heads, uint32_t 
 // tiles, which costs a merge: the run with the least estimated time, from (us,
 // measured) 8 + 5 per key tile of the longest run (head_dim 64: 5 + 2.8), and for
 // the merge 5 + 1.3 per 8 pieces of a q tile. Calls that the f32 kernel is
-// estimated to finish within 1.3 times that take it (over 155 shapes of 1 to 300
-// heads, 9 to 1024 tokens and 0 to 16000 keys before them no call is then slower
-// than under the f32 kernel alone; with 1.1, three were): with 16 / 8 heads of 128,
-// us, f32 kernel against this one, 64 tokens at 2000 22.6 / 36.6, 300 at 448 27 /
-// 33, 512 at 448 52 / 38, 300 at 2000 93 / 51, 200 at 16000 403 / 168.
+// estimated to finish within 1.3 times that take it (1.1 times with more kv heads than
+// half the CUs). Over 1495 drawn shapes of 1 to 128 kv heads, 8 to 2047 tokens and 0 to
+// 16000 keys before them, of 10 to 150 us, both kernels timed: the one taken is 1.02
+// times the better one in the mean; 61 calls are more than 3% slower than on the f32
+// kernel, 24 of them more than 10%, and 94 stay on it that this one does in less than
+// 0.9 of its time. A smaller margin or estimates fitted to these times trade one
+// against the other. With 16 / 8 heads of 128, us, f32 kernel against this one, 64
+// tokens at 2000 22.6 / 36.6, 300 at 448 27 / 33, 512 at 448 52 / 38, 300 at 2000 93 /
+// 51, 200 at 16000 403 / 168.
 PrefillPlan prefill_plan(uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim,
                          uint32_t n_queries, uint32_t pos0) {
   PrefillPlan p{};

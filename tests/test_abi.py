@@ -196,10 +196,14 @@ def test_prefill_of_many_kv_heads_needs_no_partials_of_its_own():
                     assert need == 0, (Hkv, g, n, pos0)
 
 
-def test_short_chunks_of_many_kv_heads_take_the_f32_kernel():
-    # Two rounds of workgroups with one or two short q tiles each: the f32 kernel's
-    # smaller items are done sooner (a third, measured).
+def test_short_chunks_of_many_q_tiles_take_the_f32_kernel():
+    # A few more workgroups than CUs, or two rounds of them with one or two short q
+    # tiles each: the f32 kernel's smaller items are done sooner (up to a third of the
+    # time, measured).
     L = _lib.lib()
+    for H, Hkv, d, n, pos0 in [(96, 12, 128, 230, 0), (80, 10, 128, 289, 0),
+                               (80, 16, 128, 242, 0), (350, 70, 128, 84, 12)]:
+        assert L.flock_prefill_schedule(H, Hkv, d, n, pos0) == 0, (H, Hkv, d, n, pos0)
     for H, Hkv, d, n, pos0 in [(300, 300, 128, 1, 97), (771, 257, 64, 1, 103),
                                (256, 256, 128, 33, 342), (1542, 257, 64, 41, 0),
                                (258, 129, 128, 65, 0), (1200, 200, 64, 106, 0)]:
