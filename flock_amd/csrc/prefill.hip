@@ -10,9 +10,9 @@
 // Arithmetic. f32 MFMAs run at 1/16 of the bf16 rate, so every operand is
 // split into three bf16 parts that add up to it exactly, and a product takes
 // six v_mfma_f32_32x32x16_bf16 (products of parts are exact in f32, sums are
-// f32): 2.67 times the f32 rate. What is left out is at most 2^-26 of a
-// product, below f32's own rounding; and an accumulator is rounded 6 times per
-// 16 products instead of 16.
+// f32): 2.67 times the f32 rate. What is left out is at most 2^-24 of a
+// product, half an ulp of it in f32 (of most significands below 2^-26); and an
+// accumulator is rounded 6 times per 16 products instead of 16.
 //
 // Per 64-key tile, each of 8 waves owns 32 rows and one half (32 keys) of the
 // tile; the two halves of a row keep separate online-softmax states and are

@@ -77,8 +77,9 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&s)[3]) {
 }
 
 // acc += sum over k of a[k] b[k] with both operands in three parts: the six
-// products of at least 2^-18 of the whole, smallest first. The three left out
-// are at most 2^-26 of |a| |b| together.
+// largest products, smallest first. A second part is at most
+// 2^-8 of the value and a third 2^-17, so the three products left out are at most
+// 2^-24 of |a| |b| together.
 __device__ __forceinline__ void mfma_split(floatx16& acc, const uint32x4 (&a)[3],
                                            const uint32x4 (&b)[3]) {
   auto mul = [&](int i, int j) {

@@ -1017,7 +1017,8 @@ __global__ __launch_bounds__(kQ8Threads, FLK_Q8_MM_WAVES) void q8_mm_kernel(Q8Ar
 // wide-range and subnormal inputs, where a single rounding differs in a third).
 // With c = 0 that is the order's dot4: the first product rounded, the other
 // three fused (c = +0 only turns a -0 into +0, which the fold into a partial
-// that starts at +0 cannot see). So one MFMA per four columns gives 16 tokens x
+// that starts at +0 cannot see; a partial that has itself underflowed to -0 can end
+// as +0). So one MFMA per four columns gives 16 tokens x
 // 16 rows of dot4s, and the VALU keeps what the order puts outside of dot4: d0
 // + d1, the FMA with the block's scale, and the tree over the 64 lanes.
 //
@@ -1223,7 +1224,9 @@ __device__ __forceinline__ void q8_mfma_tile(uint32_t f, uint32_t n_rt, uint32_t
 // the row tiles of one token tile share its rmsnorm scales and the staging
 // pipeline. MULTI: the general walk
 // (rows of more than 64 blocks, or of a number that is no power of two);
-// otherwise every leaf is one block.
+// otherwise every leaf is one block. With NT = 4 the fused instances fill the 256
+// VGPRs: with the norm 30 (MULTI 45) of them spill, with SwiGLU 13 (37), read back
+// where a chunk is handed over, none within the matrix products.
 template <int NT, int FUSE, bool MULTI>
 __global__ __launch_bounds__(kQ8Threads, 2) void q8_mfma_kernel(Q8Args a, uint32_t n_tt) {
   constexpr int TH = kQ8Threads;

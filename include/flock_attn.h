@@ -94,7 +94,10 @@ uint64_t flk_workspace_bytes(uint32_t n_heads, uint32_t n_kv_heads, uint32_t hea
 /* Bytes one call needs. kind: FLK_CALL_DECODE (flk_attn_decode /
  * flk_decode_layer; n = n_keys), FLK_CALL_PREFILL (n = n_queries, pos0),
  * FLK_CALL_RAGGED (n = max_n_keys, n_seqs). 0 when the call needs no workspace
- * (a single-split plan) or the shape is invalid. */
+ * (a single-split plan) or the shape is invalid. flk_attn_prefill also accepts
+ * less (down to none) where that holds the partials of its f32 kernel: the call
+ * then takes that kernel, which is slower and rounds its sums in another order.
+ * So its speed and its last bits depend on which of the two fits. */
 enum { FLK_CALL_DECODE = 0, FLK_CALL_PREFILL = 1, FLK_CALL_RAGGED = 2 };
 uint64_t flk_call_workspace_bytes(int32_t kind, uint32_t n_heads, uint32_t n_kv_heads,
                                   uint32_t head_dim, uint32_t n, uint32_t pos0, uint32_t n_seqs);
@@ -166,7 +169,8 @@ int32_t flk_attn_decode(const float* q, const float* kcache, const float* vcache
  * keys [0, pos0 + i]; the chunk's own rows must already be in the cache.
  * Tiled flash attention on the matrix cores in f32 precision (operands in
  * three bf16 parts; fp32 MFMA for calls of little work), cut over keys where
- * whole q tiles would leave the GPU idle. Range: rows whose q or output holds
+ * whole q tiles would leave the GPU idle. o may lie over q (the call then
+ * takes the fp32 kernel if ws holds its partials). Range: rows whose q or output holds
  * an infinity, a NaN or extreme magnitudes (q from 2^100 or below 2^-110, an
  * output below 2^-108) are formed in plain f32, slowly. A weight below 2^-110
  * of its row's largest is off by up to 2^-134 of that, and a v below 2^-134
