@@ -88,10 +88,9 @@ sys.path.insert(0, ROOT)
 
 METRIC = "decode-attn HBM GB/s (% peak) @32k ctx; prefill-attn TFLOP/s (% MFMA peak) @2k"
 HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
-# MI355X dense fp32 matrix. Prefill attention forms each f32 product from six
-# bf16 ones (2.5 PFLOP/s), whose own ceiling is 417 TFLOP/s: fractions of this
-# peak can pass 1.
-FP32_MFMA_PEAK_TFLOPS = 157.3
+FP32_MFMA_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix
+# Prefill attention forms each f32 product from six bf16 ones (2.5 PFLOP/s dense).
+SPLIT_MFMA_PEAK_TFLOPS = 2500 / 6
 # MI355X's published fp32 vector peak; VALU rooflines divide by it. It counts
 # packed-fp32 instructions (two flops per lane per cycle), which this library
 # never emits, so its VALU code can reach at most half of it: VALU rooflines
@@ -129,6 +128,7 @@ class Workload:
     name = ""
     unit = "GB/s"
     bound = "hbm"
+    mfma_peak = FP32_MFMA_PEAK_TFLOPS  # of the matrix instructions a "mfma" workload uses
     calls_per_step = 1
     graph_step = False  # step() replays a captured graph: call time = step time / calls
     roofline_note = None
@@ -148,7 +148,7 @@ class Workload:
             peak, unit, key = FP32_VECTOR_PEAK_TFLOPS, "TFLOP/s", "flops_per_launch"
         else:
             achieved = self.work_per_call / (call_ms * 1e-3) / 1e12
-            peak, unit, key = FP32_MFMA_PEAK_TFLOPS, "TFLOP/s", "flops_per_launch"
+            peak, unit, key = round(self.mfma_peak, 1), "TFLOP/s", "flops_per_launch"
         out = {"bound": self.bound, "achieved": round(achieved, 2), "peak": peak, "unit": unit,
                "frac": round(achieved / peak, 4), "traffic": traffic, "kernel": self.kernel,
                key: self.work_per_call, "avg_launch_us": round(call_ms * 1e3, 2)}
@@ -380,9 +380,9 @@ class Prefill2k(Workload):
     unit = "TFLOP/s"
     bound = "mfma"
     kernel = "flk_attn_prefill: prefill_kernel<128> (equal runs of key tiles + prefill_merge_kernel)"
-    roofline_note = ("each f32 product is six bf16 MFMA ones, whose ceiling is 417 TFLOP/s: the "
-                     "fraction of the fp32 MFMA peak can pass 1; traffic was counted on the f32 "
-                     "kernel, before partials of cut q tiles")
+    mfma_peak = SPLIT_MFMA_PEAK_TFLOPS
+    roofline_note = ("peak: f32 products, each of six bf16 MFMA ones (2.5 PFLOP/s / 6); "
+                     "frac_of_fp32_mfma_peak, against 157.3 TFLOP/s, can pass 1")
 
     def __init__(self, torch, ops, n=2048, pos0=0, layers=1):
         self.torch, self.ops = torch, ops
@@ -513,7 +513,7 @@ class Prefill2k(Workload):
 
 class Chunk32k(Prefill2k):
     name = "chunk32k"
-    kernel = "flk_attn_prefill: prefill_kernel<128> (key splits) + prefill_merge_kernel<128>"
+    kernel = "flk_attn_prefill: prefill_kernel<128> (equal runs of key tiles) + prefill_merge_kernel"
 
     def __init__(self, torch, ops):
         super().__init__(torch, ops, n=64, pos0=32768, layers=28)
@@ -812,7 +812,9 @@ class Q8Prefill(Workload):
 
     name = "q8prefill"
     unit = "TFLOP/s"
-    bound = "valu"
+    bound = "mfma"
+    roofline_note = ("f32 MFMAs form the dot4s of the exact summation order; the rest of the order "
+                     "(two VALU operations per MFMA output) overlaps with them only in part")
     kernel = "flk_q8_gate_up_swiglu: q8_mfma_kernel<4, kMmNorm> (64 rows x 64 tokens per tile)"
     n_tokens, ffn, hid = 2048, 3072, 1024
 
@@ -1248,6 +1250,7 @@ def main():
         if main_res["unit"] == "GB/s":
             out["frac_of_hbm_peak"] = round(main_res["value"] / HBM_PEAK_GBS, 4)
         elif main_res["unit"] == "TFLOP/s" and main_res["roofline"]["bound"] == "mfma":
+            out["frac_of_mfma_peak"] = round(main_res["value"] / main_res["roofline"]["peak"], 4)
             out["frac_of_fp32_mfma_peak"] = round(main_res["value"] / FP32_MFMA_PEAK_TFLOPS, 4)
         elif main_res["unit"] == "TFLOP/s":
             out["frac_of_fp32_vector_peak"] = round(main_res["value"] / FP32_VECTOR_PEAK_TFLOPS, 4)
@@ -1271,6 +1274,7 @@ def main():
                 if res["unit"] == "GB/s":
                     res["frac_of_hbm_peak"] = round(res["value"] / HBM_PEAK_GBS, 4)
                 elif res["unit"] == "TFLOP/s" and b == "mfma":
+                    res["frac_of_mfma_peak"] = round(res["value"] / res["roofline"]["peak"], 4)
                     res["frac_of_fp32_mfma_peak"] = round(res["value"] / FP32_MFMA_PEAK_TFLOPS, 4)
                 out[key] = res
                 secondary.append((key, name, cpu))
