@@ -177,7 +177,7 @@ uint64_t flk_workspace_bytes(uint32_t n_heads, uint32_t n_kv_heads, uint32_t hea
   const DecodeShape ds1{n_heads, n_kv_heads, head_dim, 1, max_keys};
   const uint64_t d1 = decode_ws_bound(ds1);
   if (d1 > need) need = d1;
-  if (max_queries > 0) {
+  if (max_queries > 0 && n_heads / n_kv_heads <= 8) {  // larger groups are refused
     const uint32_t nq = max_queries < max_keys ? max_queries : max_keys;
     const uint64_t b = prefill_ws_bound(n_heads, n_kv_heads, head_dim, nq, max_keys);
     if (b > need) need = b;
@@ -195,6 +195,7 @@ uint64_t flk_call_workspace_bytes(int32_t kind, uint32_t n_heads, uint32_t n_kv_
     case FLK_CALL_RAGGED:
       return decode_ws_bytes(DecodeShape{n_heads, n_kv_heads, head_dim, n_seqs ? n_seqs : 1, n});
     case FLK_CALL_PREFILL:
+      if (n_heads / n_kv_heads > 8) return 0;
       return prefill_ws_bytes(prefill_plan(n_heads, n_kv_heads, head_dim, n, pos0), head_dim);
     default:
       return 0;

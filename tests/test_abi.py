@@ -210,6 +210,18 @@ def test_short_chunks_of_many_q_tiles_take_the_f32_kernel():
         assert L.flock_prefill_schedule(H, Hkv, d, n, pos0) == 0, (H, Hkv, d, n, pos0)
 
 
+@pytest.mark.parametrize("H,Hkv", [(9, 1), (65, 1), (128, 1), (256, 1), (600, 2)])
+def test_workspace_queries_of_groups_that_calls_refuse(H, Hkv):
+    # No q tile holds a group of more than 64 rows: the sizes of such shapes divided
+    # by zero. flk_attn_prefill refuses groups of more than 8.
+    L = _lib.lib()
+    assert L.flk_call_workspace_bytes(1, H, Hkv, 128, 100, 0, 1) == 0
+    assert L.flk_workspace_bytes(H, Hkv, 128, 2048, 100, 1) == \
+        L.flk_workspace_bytes(H, Hkv, 128, 2048, 0, 1)
+    assert L.flk_attn_prefill(FAKE, FAKE, FAKE, FAKE, H, Hkv, 128, 100, 0, FAKE,
+                              1 << 40) == _lib.FLK_ERR_UNSUPPORTED
+
+
 def test_ragged_workspace_bound():
     L = _lib.lib()
     for seqs in (1, 3, 64, 200):
